@@ -177,6 +177,34 @@ def test_gemm_k_order_classes_are_bitwise_identical(device, epi):
                 assert torch.equal(out, outs[0]), f"class {cls}: plan {plan} differs from plan {plans[0]}"
 
 
+@pytest.mark.parametrize("dt", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("plan", [33, 34, 35])
+def test_gemm_panel_plans(device, dt, plan):
+    """Panel-ring tiles: one K tile, odd and even counts of them, ragged M
+    and N below, at and past a tile, every epilogue; against fp64 and, bit for
+    bit, against class-1 plan 9 (which sums the same 16-deep products in the
+    same order with 32 x 32 MFMAs)."""
+    g = _gen(77 + plan)
+    for m, n, k in ((1, 4, 64), (129, 132, 128), (256, 256, 192), (385, 260, 1088)):
+        a = torch.randn(m, k, generator=g).to(dt).to(device)
+        w = (torch.randn(n, k, generator=g) / math.sqrt(k)).to(dt).to(device)
+        b = torch.randn(n, generator=g).to(dt).to(device)
+        r0 = torch.randn(m, n, generator=g).to(device)
+        x = torch.randn(m + 3, n, generator=g).to(dt).to(device)
+        rows = torch.randperm(m + 3, generator=g)[:m].int().to(device)
+        for epi in (ops.EPI_BIAS, ops.EPI_BIAS_GELU, ops.EPI_BIAS_RESIDUAL):
+            _gemm_case(device, m, n, k, dt, epi, plan)
+            outs = []
+            for p in (9, plan):
+                out = r0.clone() if epi == ops.EPI_BIAS_RESIDUAL else torch.zeros(m, n, dtype=dt, device=device)
+                outs.append(ops.gemm(a, w, b, out, epi, p))
+            torch.cuda.synchronize()
+            assert torch.equal(*outs), (m, n, k, epi)
+        outs = [ops.gemm_residual_from(a, w, b, torch.zeros(m, n, device=device), x, rows, plan=p) for p in (9, plan)]
+        torch.cuda.synchronize()
+        assert torch.equal(*outs), (m, n, k, "from")
+
+
 @pytest.mark.parametrize("epi", [ops.EPI_BIAS, ops.EPI_BIAS_GELU, ops.EPI_BIAS_RESIDUAL])
 @pytest.mark.parametrize("plan", [9, 14, 16, 21, 29])
 def test_gemm_write_through_launch_equals_plain(device, epi, plan):

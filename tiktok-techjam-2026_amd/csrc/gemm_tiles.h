@@ -198,49 +198,63 @@ struct ResPrefetch {
   }
 };
 
-// The bias pieces of a wave's columns nw.. (the epilogue's layout: lane
-// (l32, hi) needs columns nw + 32 i + 8 g + 4 hi .. +3), raw.  All loads go
+// The bias pieces of a wave's columns nw.. (the epilogue's layout: with
+// 32 x 32 accumulator blocks lane (l32, hi) needs columns nw + 32 i + 8 g +
+// 4 hi .. +3, with 16 x 16 ones (M16) lane (l16, q) columns nw + 32 i + 16 g +
+// 4 q .. +3, g < 2), raw.  All loads go
 // out before any is used -- one memory round trip; a load under a per-lane
 // condition would be waited for on its own, one round trip per load -- with
 // columns past N clamped into range (N % 4 == 0, N >= 4) and zeroed when
 // converted.  A kernel whose registers allow it loads them before its main
 // loop, which takes that round trip off the end of the launch.
-template <typename T, int FN>
+template <typename T, int FN, bool M16 = false>
 struct BiasRaw {
   typedef typename Quad<T>::raw Raw;
-  Raw r[FN][4];
+  static constexpr int NG = M16 ? 2 : 4;  // pieces per 32 columns
+  Raw r[FN][NG];
+  // this lane's first column of piece (i, g), relative to nw
+  static __device__ __forceinline__ int col(int i, int g, int lane) {
+    return M16 ? i * 32 + g * 16 + (lane >> 4) * 4 : i * 32 + g * 8 + (lane >> 5) * 4;
+  }
   __device__ __forceinline__ void load(const T* __restrict__ bias, int N, int nw, int lane) {
-    const int hi = lane >> 5;
 #pragma unroll
     for (int i = 0; i < FN; ++i)
 #pragma unroll
-      for (int g = 0; g < 4; ++g) r[i][g] = Raw{};
+      for (int g = 0; g < NG; ++g) r[i][g] = Raw{};
     if (bias != nullptr) {
 #pragma unroll
       for (int i = 0; i < FN; ++i)
 #pragma unroll
-        for (int g = 0; g < 4; ++g)
-          r[i][g] = *reinterpret_cast<const Raw*>(bias + min(nw + i * 32 + g * 8 + hi * 4, N - 4));
+        for (int g = 0; g < NG; ++g)
+          r[i][g] = *reinterpret_cast<const Raw*>(bias + min(nw + col(i, g, lane), N - 4));
     }
   }
 };
+
+// The accumulators of a wave's (32 FM) x (32 FN) block as the kernels hold
+// them: C^T blocks of 32 x 32 (f32x16, [FN][FM]) or of 16 x 16 (f32x4,
+// [2 FN][2 FM]; lane (l16, q) of block (i, j) owns columns 16 i + 4 q .. +3
+// of row 16 j + l16).
+template <int FM, int FN> using Acc32 = f32x16[FN][FM];
+template <int FM, int FN> using Acc16 = f32x4[2 * FN][2 * FM];
 
 // Stores this wave's (32 FM) x (32 FN) block at rows mw.., columns nw.. of
 // C (rows >= M and columns >= N dropped).  `stage` is the wave's private
 // EpiStage<T, EPI, FN>::BYTES of LDS.  `bpre`, when given, holds the bias
 // pieces already loaded (BiasRaw::load with the same bias, N, nw, lane).
 // RB_: residual pieces per batched read (0: read one by one).
-template <typename T, int EPI, int FM, int FN, typename Pre = NoPrefetch, int RB_ = kResBatch>
-__device__ __forceinline__ void epilogue(const f32x16 (&acc)[FN][FM], const T* __restrict__ bias,
-                                         void* __restrict__ Cv, int64_t ldc, int M, int N, int mw, int nw,
-                                         int lane, char* __restrict__ stage, const Pre& pre = Pre(),
-                                         const BiasRaw<T, FN>* bpre = nullptr,
-                                         const ResSrc& src = ResSrc{nullptr, 0, nullptr, 0, nullptr}) {
+template <typename T, int EPI, int FM, int FN, typename Pre = NoPrefetch, int RB_ = kResBatch, bool M16 = false>
+__device__ __forceinline__ void epilogue(
+    const typename std::conditional<M16, Acc16<FM, FN>, Acc32<FM, FN>>::type& acc, const T* __restrict__ bias,
+    void* __restrict__ Cv, int64_t ldc, int M, int N, int mw, int nw, int lane, char* __restrict__ stage,
+    const Pre& pre = Pre(), const typename std::common_type<BiasRaw<T, FN, M16>>::type* bpre = nullptr,
+    const ResSrc& src = ResSrc{nullptr, 0, nullptr, 0, nullptr}) {
+  typedef BiasRaw<T, FN, M16> Bias;
   typedef EpiStage<T, EPI, FN> E;
   constexpr int LPR = E::LPR;          // 16-byte pieces per staged row
   constexpr int NPC = 32 * LPR;        // pieces per 32-row block
   constexpr int NIT = (NPC + 63) / 64; // read instructions per block
-  const int l32 = lane & 31, hi = lane >> 5;
+  const int l32 = lane & 31, hi = lane >> 5, l16 = lane & 15, q16 = lane >> 4;
   // 16-byte output pieces need a 16-byte aligned C and a leading dimension
   // that keeps every row 16-byte aligned; otherwise pieces go out as halves.
   const bool a16 = ((uintptr_t)Cv & 15) == 0 && (ldc % E::SV) == 0;
@@ -248,22 +262,27 @@ __device__ __forceinline__ void epilogue(const f32x16 (&acc)[FN][FM], const T* _
   const bool wt = (int64_t)M * N * OB >= kWtMinBytes;
 
   // bias of this wave's columns (loaded here unless the caller did)
-  BiasRaw<T, FN> own;
+  Bias own;
   if (bpre == nullptr) own.load(bias, N, nw, lane);
-  const BiasRaw<T, FN>& braw = bpre != nullptr ? *bpre : own;
-  float4 bv[FN][4];
+  const Bias& braw = bpre != nullptr ? *bpre : own;
+  float4 bv[FN][Bias::NG];
 #pragma unroll
   for (int i = 0; i < FN; ++i)
 #pragma unroll
-    for (int g = 0; g < 4; ++g) {
-      const int n = nw + i * 32 + g * 8 + hi * 4;
-      bv[i][g] = n < N ? Quad<T>::to(braw.r[i][g]) : make_float4(0.f, 0.f, 0.f, 0.f);
-    }
+    for (int g = 0; g < Bias::NG; ++g)
+      bv[i][g] = nw + Bias::col(i, g, lane) < N ? Quad<T>::to(braw.r[i][g]) : make_float4(0.f, 0.f, 0.f, 0.f);
 
-  // columns 32 i + 8 g + 4 hi .. +3 of this lane's row, bias / GELU applied
-  auto value = [&](int j, int i, int g) __attribute__((always_inline)) {
-    float4 v = make_float4(acc[i][j][4 * g + 0] + bv[i][g].x, acc[i][j][4 * g + 1] + bv[i][g].y,
-                           acc[i][j][4 * g + 2] + bv[i][g].z, acc[i][j][4 * g + 3] + bv[i][g].w);
+  // columns Bias::col(i, g) .. +3 of this lane's row of 32-row block j (of
+  // its 16-row half s with 16 x 16 accumulators), bias / GELU applied
+  auto value = [&](int j, int i, int g, int s = 0) __attribute__((always_inline)) {
+    float4 v;
+    if constexpr (M16) {
+      const f32x4& a = acc[2 * i + g][2 * j + s];
+      v = make_float4(a[0] + bv[i][g].x, a[1] + bv[i][g].y, a[2] + bv[i][g].z, a[3] + bv[i][g].w);
+    } else {
+      v = make_float4(acc[i][j][4 * g + 0] + bv[i][g].x, acc[i][j][4 * g + 1] + bv[i][g].y,
+                      acc[i][j][4 * g + 2] + bv[i][g].z, acc[i][j][4 * g + 3] + bv[i][g].w);
+    }
     if (EPI == TJK_EPI_BIAS_GELU) {
       v.x = gelu_erf(v.x); v.y = gelu_erf(v.y); v.z = gelu_erf(v.z); v.w = gelu_erf(v.w);
     }
@@ -273,9 +292,11 @@ __device__ __forceinline__ void epilogue(const f32x16 (&acc)[FN][FM], const T* _
   // Staging offsets, the same for every 32-row block.  Writes: piece C + hi
   // of row l32 (C even, a compile-time value) sits at C ^ wx with
   // wx = x(l32) ^ hi, i.e. at the constant C & ~(G - 1) plus one of G / 2
-  // per-lane offsets.  Reads: one offset per read instruction.
-  char* const wrow = stage + l32 * LPR * 16;
-  const int wx = E::x(l32) ^ hi;
+  // per-lane offsets.  Reads: one offset per read instruction.  (16 x 16
+  // accumulators: row l16 of a 16-row half, piece C + b with C % 4 == 0 and b
+  // the lane's two low bits; 16 rows on, x is the same.)
+  char* const wrow = stage + (M16 ? l16 : l32) * LPR * 16;
+  const int wx = M16 ? E::x(l16) ^ (E::SV == 4 ? q16 : 2 * (q16 & 1) + (q16 >> 1)) : E::x(l32) ^ hi;
   auto wslot = [&](int c) __attribute__((always_inline)) {
     return wrow + 16 * ((c & ~(E::G - 1)) + ((c & (E::G - 1)) ^ wx));
   };
@@ -347,7 +368,24 @@ __device__ __forceinline__ void epilogue(const f32x16 (&acc)[FN][FM], const T* _
     res_read(0);
 #pragma unroll
     for (int i = 0; i < FN; ++i) {
-      if constexpr (E::SV == 4) {  // fp32 staged: a lane's four columns are one piece
+      if constexpr (M16) {
+#pragma unroll
+        for (int s = 0; s < 2; ++s) {
+          if constexpr (E::SV == 4) {
+#pragma unroll
+            for (int g = 0; g < 2; ++g)
+              *reinterpret_cast<float4*>(wslot(8 * i + 4 * g) + s * 256 * LPR) = value(j, i, g, s);
+          } else {
+            // rows of 16 lanes trade halves: lane (l16, q) ends with the two
+            // adjacent quads 2 (q / 2), 2 (q / 2) + 1 of block 2 i + q % 2
+            const typename Quad<T>::raw x = Quad<T>::from(value(j, i, 0, s));
+            const typename Quad<T>::raw y = Quad<T>::from(value(j, i, 1, s));
+            const auto s0 = __builtin_amdgcn_permlane16_swap(x.x, y.x, false, false);
+            const auto s1 = __builtin_amdgcn_permlane16_swap(x.y, y.y, false, false);
+            *reinterpret_cast<uint4*>(wslot(4 * i) + s * 256 * LPR) = make_uint4(s0[0], s1[0], s0[1], s1[1]);
+          }
+        }
+      } else if constexpr (E::SV == 4) {  // fp32 staged: a lane's four columns are one piece
 #pragma unroll
         for (int g = 0; g < 4; ++g) *reinterpret_cast<float4*>(wslot(8 * i + 2 * g)) = value(j, i, g);
       } else {
@@ -711,6 +749,214 @@ __device__ __forceinline__ void dtl_accumulate(
   // tile) has landed and every wave is done reading.
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
   __syncthreads();
+}
+
+// ------------------------------------------------------- panel-ring GEMM
+//
+// Main loop for the largest tiles: 2 x 2 waves with (32 FM) x (32 FN) wave
+// tiles, one wave per SIMD, accumulators in all 256 AGPRs (FM = FN = 4).
+// What bounds these launches on MI355X is power: the matrix pipe is busy
+// ~90% of the main loop's cycles while the clock sits at 1.5-1.7 GHz, so the
+// loop is built to spend less energy per product and to keep the pipe fed:
+//   * 16x16x32 MFMAs: one instruction contracts 32 of K, so an accumulator
+//     is read and written half as often per product as with 32x32x16.  The
+//     MFMAs alone ran at 2.19 GHz against 1.89 GHz (same probe, 256 x 256
+//     tiles of 8192^3).  They are written in inline asm with the accumulator
+//     tied to one register: the builtin's separate source and destination
+//     made the compiler copy accumulators around every MFMA.
+//   * The K tile (64 deep) of A and of W is split into two panels each: A
+//     panel h holds each wave row's 32-row blocks of half h, W panel g each
+//     wave column's.  A step multiplies one A panel by one W panel out of
+//     registers while it reads one further panel's fragments from LDS, so a
+//     panel's LDS slot is free again one step after it was read and its next
+//     K tile's DMA goes out then, a quarter of a tile per step.  A 2-slot
+//     ring whose slot frees only at the end of a K tile has to issue the
+//     whole tile's DMA at once and stalls the waves' in-order MFMAs.
+//   * Steps run (A0,Wx) (A0,Wy) (A1,Wy) (A1,Wx), x = t & 1 for K tile t, so
+//     each step needs one new panel and no fragment register is overwritten
+//     while in use.  Panels are read in the order A0, Wx, Wy, A1 of each K
+//     tile; the step that reads panel v (of that sequence) issues the DMA of
+//     panel v + 7 into the slot of panel v - 1 and ends waiting for panel
+//     v + 1: six panels stay in flight.
+//   * Fragment reads go in the first half of a step, its DMA between 5/8
+//     and 7/8 of it: measured on 8192^3, 2303 cycles per K tile (2048 of
+//     them MFMA) against 2412 with the DMA spread evenly and 2483 with it
+//     first.
+// K need not be a multiple of 64: 16-byte pieces past K point outside the
+// buffer range and arrive as zeros, like rows past M or N.  An odd number
+// of K tiles runs one more, of zeros.
+enum { kPanelA0 = 0, kPanelA1 = 1, kPanelW0 = 2, kPanelW1 = 3 };
+
+template <int V> using IntC = std::integral_constant<int, V>;
+
+template <int FM, int FN>
+struct PanelGeom {
+  static constexpr int BM = 64 * FM, BN = 64 * FN;
+  static constexpr int F[4] = {(FM + 1) / 2, FM / 2, (FN + 1) / 2, FN / 2};  // 32-row blocks per wave of a panel
+  static constexpr int OFF[4] = {0, F[0] * 8192, BM * 128, BM * 128 + F[2] * 8192};  // bytes in a slot
+  static constexpr int SLOT = (BM + BN) * 128;
+  static constexpr int ND[4] = {F[0] * 2, F[1] * 2, F[2] * 2, F[3] * 2};  // DMA instructions per wave
+  static constexpr int ALL = 2 * (ND[0] + ND[1] + ND[2] + ND[3]);         // both slots
+  static constexpr int LDS = 2 * SLOT;
+  static_assert(FM >= 2 && FN >= 2 && ALL <= 63, "two panels per operand; vmcnt range");
+};
+
+template <typename T> __device__ __forceinline__ void mma16_tied(f32x4& c, const typename Mfma<T>::frag& a,
+                                                                 const typename Mfma<T>::frag& b) {
+  if constexpr (std::is_same<T, bf16>::value)
+    asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+a"(c) : "v"(a), "v"(b));
+  else
+    asm volatile("v_mfma_f32_16x16x32_f16 %0, %1, %2, %0" : "+a"(c) : "v"(a), "v"(b));
+}
+
+// Buffer descriptor (stride 0, raw dwords) over `bytes` bytes of a
+// wave-uniform address, for lds_dma16.
+__device__ __forceinline__ u32x4 lds_dma_rsrc(const void* p, int64_t bytes) {
+  const uint64_t a = (uint64_t)(uintptr_t)p;
+  const int n = (int)(bytes > 0x7fffffff ? 0x7fffffff : bytes);
+  return u32x4{(uint32_t)__builtin_amdgcn_readfirstlane((uint32_t)a),
+               (uint32_t)__builtin_amdgcn_readfirstlane((uint32_t)(a >> 32)) & 0xffffu,
+               (uint32_t)__builtin_amdgcn_readfirstlane(n), 0x00020000u};
+}
+// One LDS DMA: each lane copies 16 bytes at voff of the descriptor's range
+// (zeros past it) to LDS byte lds_addr + 16 * lane.  Inline asm, so that the
+// compiler does not wait for copies in flight before LDS reads; the caller's
+// s_waitcnt vmcnt and s_barrier order them.
+__device__ __forceinline__ void lds_dma16(u32x4 rsrc, uint32_t voff, uint32_t lds_addr) {
+  asm volatile("buffer_load_dwordx4 %0, %1, 0 offen lds" ::"v"(voff), "s"(rsrc), "{m0}"(lds_addr));
+}
+
+// acc += A[m0 : m0 + 64 FM, :] W[n0 : n0 + 64 FN, :]^T for this wave's
+// sub-tile.  On return every DMA has landed and the workgroup has met at a
+// barrier, so the LDS ring may be reused.
+template <typename T, int FM, int FN>
+__device__ __forceinline__ void panel_accumulate(char* smem, const T* __restrict__ A, int64_t lda,
+                                                 const T* __restrict__ W, int64_t ldw, int M, int N, int K, int m0,
+                                                 int n0, Acc16<FM, FN>& acc) {
+  typedef PanelGeom<FM, FN> G;
+  typedef typename Mfma<T>::frag Frag;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wm = wave >> 1, wn = wave & 1, l16 = lane & 15, q16 = lane >> 4;
+  const u32x4 rsa = lds_dma_rsrc(A + (int64_t)m0 * lda, (int64_t)min(G::BM, M - m0) * lda * (int64_t)sizeof(T));
+  const u32x4 rsw = lds_dma_rsrc(W + (int64_t)n0 * ldw, (int64_t)min(G::BN, N - n0) * ldw * (int64_t)sizeof(T));
+  const uint32_t lds0 = (uint32_t)(uintptr_t)(lds_void*)smem;
+  // DMA instruction i of a panel fills its rows 32 i + 8 wave .. + 7 (128 B
+  // each); lane l lands in row l / 8, physical chunk l % 8, so it fetches
+  // logical chunk (l % 8) ^ swz(row).
+  const int line0 = wave * 8 + lane / 8;
+  const uint32_t lcb = (uint32_t)(((lane & 7) ^ swz<128>(line0)) << 4);
+  const uint32_t kend = (uint32_t)K * (uint32_t)sizeof(T);
+  const uint32_t lab = (uint32_t)(lda * (int64_t)sizeof(T)), lwb = (uint32_t)(ldw * (int64_t)sizeof(T));
+  // tile row of panel row 32 i + line0: the panel's rows are each wave row's
+  // (column's) F blocks in turn
+  auto row_of = [&](int p, int i) __attribute__((always_inline)) {
+    const int f = G::F[p], line = i * 32 + line0, w = line / (32 * f), r = line % (32 * f);
+    return w * 32 * (p < 2 ? FM : FN) + (p & 1 ? 32 * G::F[p - 1] : 0) + r;
+  };
+  uint32_t va0[G::ND[0]], va1[G::ND[1]], vw0[G::ND[2]], vw1[G::ND[3]];
+#pragma unroll
+  for (int i = 0; i < G::ND[0]; ++i) va0[i] = row_of(kPanelA0, i) * lab + lcb;
+#pragma unroll
+  for (int i = 0; i < G::ND[1]; ++i) va1[i] = row_of(kPanelA1, i) * lab + lcb;
+#pragma unroll
+  for (int i = 0; i < G::ND[2]; ++i) vw0[i] = row_of(kPanelW0, i) * lwb + lcb;
+#pragma unroll
+  for (int i = 0; i < G::ND[3]; ++i) vw1[i] = row_of(kPanelW1, i) * lwb + lcb;
+  // instruction i of panel P of K tile kt into slot S
+  auto dma = [&](auto P, auto S, int kt, int i) __attribute__((always_inline)) {
+    constexpr int p = decltype(P)::value, s = decltype(S)::value;
+    const uint32_t kb = (uint32_t)kt * 128u;
+    const uint32_t ko = kb + lcb < kend ? kb : (uint32_t)kPastEnd;
+    const uint32_t v = p == kPanelA0 ? va0[i] : p == kPanelA1 ? va1[i] : p == kPanelW0 ? vw0[i] : vw1[i];
+    lds_dma16(p < 2 ? rsa : rsw, v + ko, lds0 + s * G::SLOT + G::OFF[p] + (i * 4 + wave) * 1024);
+  };
+  // Fragments of a panel: its 16-row blocks x two 32-deep steps; lane
+  // (l16, q16) holds row l16, K elements 8 q16 .. + 7 of the step.
+  Frag fa0[2 * G::F[0]][2], fa1[2 * G::F[1]][2], fw0[2 * G::F[2]][2], fw1[2 * G::F[3]][2];
+  const int sw = swz<128>(l16);
+  const char* const ra0 = smem + G::OFF[0] + (wm * 32 * G::F[0] + l16) * 128;
+  const char* const ra1 = smem + G::OFF[1] + (wm * 32 * G::F[1] + l16) * 128;
+  const char* const rw0 = smem + G::OFF[2] + (wn * 32 * G::F[2] + l16) * 128;
+  const char* const rw1 = smem + G::OFF[3] + (wn * 32 * G::F[3] + l16) * 128;
+  auto read = [&](auto P, auto S, int r) __attribute__((always_inline)) {
+    constexpr int p = decltype(P)::value, s = decltype(S)::value;
+    const char* const b = (p == kPanelA0 ? ra0 : p == kPanelA1 ? ra1 : p == kPanelW0 ? rw0 : rw1) + s * G::SLOT;
+    const Frag f = *reinterpret_cast<const Frag*>(b + (r >> 1) * 2048 + (((4 * (r & 1) + q16) ^ sw) << 4));
+    if constexpr (p == kPanelA0) fa0[r >> 1][r & 1] = f;
+    else if constexpr (p == kPanelA1) fa1[r >> 1][r & 1] = f;
+    else if constexpr (p == kPanelW0) fw0[r >> 1][r & 1] = f;
+    else fw1[r >> 1][r & 1] = f;
+  };
+  // One step: the MFMAs of A panel h x W panel g; reads panel RP from slot
+  // RS, issues the DMA of panel DP of K tile dkt into slot DS; XP is the
+  // panel the next step reads.
+  auto step = [&](auto H, auto Gn, auto RP, auto RS, auto DP, auto DS, int dkt, auto XP) __attribute__((always_inline)) {
+    constexpr int h = decltype(H)::value, g = decltype(Gn)::value, rp = decltype(RP)::value, dp = decltype(DP)::value;
+    constexpr int na = 2 * G::F[h], nw = 2 * G::F[2 + g];  // 16-row blocks
+    constexpr int NMF = na * nw * 2, NR = 4 * G::F[rp], ND = G::ND[dp];
+    constexpr int R1 = NMF / 2, D0 = NMF * 5 / 8, D1 = NMF * 7 / 8;
+#pragma unroll
+    for (int m = 0; m < NMF; ++m) {
+      const int ks = m / (na * nw), i = m % (na * nw) / na, j = m % na;
+      mma16_tied<T>(acc[(g ? 2 * G::F[2] : 0) + i][(h ? 2 * G::F[0] : 0) + j], g ? fw1[i % (2 * G::F[3])][ks] : fw0[i][ks],
+                    h ? fa1[j % (2 * G::F[1])][ks] : fa0[j][ks]);
+      if (m & 1) {
+        if (m < R1) {
+#pragma unroll
+          for (int r = m / 2 * NR / (R1 / 2); r < (m / 2 + 1) * NR / (R1 / 2); ++r) read(RP, RS, r);
+        } else if (m >= D0 && m < D1) {
+          constexpr int DN = (D1 - D0) / 2;
+#pragma unroll
+          for (int d = (m - D0) / 2 * ND / DN; d < ((m - D0) / 2 + 1) * ND / DN; ++d) dma(DP, DS, dkt, d);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    }
+    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(G::ALL - G::ND[rp] - G::ND[decltype(XP)::value]) : "memory");
+    asm volatile("s_barrier" ::: "memory");
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  constexpr IntC<0> c0{};
+  constexpr IntC<1> c1{};
+  constexpr IntC<kPanelA0> A0{};
+  constexpr IntC<kPanelA1> A1{};
+  constexpr IntC<kPanelW0> W0{};
+  constexpr IntC<kPanelW1> W1{};
+  auto dma_panel = [&](auto P, auto S, int kt) __attribute__((always_inline)) {
+#pragma unroll
+    for (int i = 0; i < G::ND[decltype(P)::value]; ++i) dma(P, S, kt, i);
+  };
+  // K tiles 0 and 1 in flight, panels 0 and 1 read, panel 8 issued
+  dma_panel(A0, c0, 0); dma_panel(W0, c0, 0); dma_panel(W1, c0, 0); dma_panel(A1, c0, 0);
+  dma_panel(A0, c1, 1); dma_panel(W1, c1, 1); dma_panel(W0, c1, 1); dma_panel(A1, c1, 1);
+  asm volatile("s_waitcnt vmcnt(%0)" ::"n"(G::ALL - G::ND[kPanelA0] - G::ND[kPanelW0]) : "memory");
+  asm volatile("s_barrier" ::: "memory");
+#pragma unroll
+  for (int r = 0; r < 4 * G::F[kPanelA0]; ++r) read(A0, c0, r);
+#pragma unroll
+  for (int r = 0; r < 4 * G::F[kPanelW0]; ++r) read(W0, c0, r);
+  asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+  asm volatile("s_barrier" ::: "memory");
+  dma_panel(A0, c0, 2);
+  asm volatile("s_waitcnt vmcnt(%0)" ::"n"(G::ALL - G::ND[kPanelW0] - G::ND[kPanelW1]) : "memory");
+  asm volatile("s_barrier" ::: "memory");
+  __builtin_amdgcn_sched_barrier(0);
+  const int nkt = (int)((kend + 127u) / 128u);
+  for (int t = 0; t < nkt; t += 2) {
+    step(c0, c0, W1, c0, W0, c0, t + 2, A1);
+    step(c0, c1, A1, c0, W1, c0, t + 2, A0);
+    step(c1, c1, A0, c1, A1, c0, t + 2, W1);
+    step(c1, c0, W1, c1, A0, c1, t + 3, W0);
+    step(c0, c1, W0, c1, W1, c1, t + 3, A1);
+    step(c0, c0, A1, c1, W0, c1, t + 3, A0);
+    step(c1, c0, A0, c0, A1, c1, t + 3, W0);
+    step(c1, c1, W0, c0, A0, c0, t + 4, W1);
+  }
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  __syncthreads();
+  // the last MFMAs' results, which the compiler does not track, are written
+  asm volatile("s_nop 15\n\ts_nop 15" ::: "memory");
 }
 
 template <typename T, int FM, int FN>
