@@ -205,6 +205,40 @@ def test_gemm_panel_plans(device, dt, plan):
         assert torch.equal(*outs), (m, n, k, "from")
 
 
+@pytest.mark.parametrize("m,n,k", [  # the tile the default rule takes:
+    (1, 4, 8), (70, 68, 200),   # 64 x 64
+    (5547, 324, 40),            # 96 x 128
+    (5923, 1300, 72),           # 192 x 128, panel ring
+    (5467, 1036, 200),          # 128 x 128, panel ring
+    (5431, 2180, 520),          # 256 x 256, panel ring
+    (5430, 3072, 1000),         # 192 x 384
+    (33, 36, 1000),             # 32 x 32, K split in 2
+    (4161, 44, 520),            # 32 x 64, K split in 2
+    (2748, 164, 520),           # 64 x 64, K split in 2
+    (5534, 136, 600),           # 128 x 64, K split in 2
+    (33, 36, 2056), (4590, 40, 2600),  # 32 x 32, 32 x 64, K split in 4
+])
+@pytest.mark.parametrize("dt", [torch.bfloat16, torch.float16])
+def test_gemm_default_tile_takes_any_k(device, dt, m, n, k):
+    """The default tile at K that is no multiple of 64, in every tile the rule
+    takes: the columns between K and the rows' pitch are NaN and must not
+    enter the sums (nor the rows past M and N, outside the buffers)."""
+    g = _gen(5 + m + n + k)
+    a = torch.full((m, k + 24), float("nan"), dtype=dt)
+    w = torch.full((n, k + 8), float("nan"), dtype=dt)
+    a[:, :k] = torch.randn(m, k, generator=g).to(dt)
+    w[:, :k] = (torch.randn(n, k, generator=g) / math.sqrt(k)).to(dt)
+    b = torch.randn(n, generator=g).to(dt)
+    r0 = torch.randn(m, n, generator=g)
+    ref = a[:, :k].to(device).double() @ w[:, :k].to(device).double().t() + b.to(device).double()
+    ad, wd, bd = a.to(device)[:, :k], w.to(device)[:, :k], b.to(device)
+    out = ops.gemm(ad, wd, bd, torch.full((m, n), float("nan"), dtype=dt, device=device), ops.EPI_BIAS)
+    res = ops.gemm(ad, wd, bd, r0.to(device), ops.EPI_BIAS_RESIDUAL)
+    torch.cuda.synchronize()
+    _close(out, ref.cpu(), OUT_RTOL[dt], 1e-4)
+    _close(res, (ref + r0.to(device).double()).cpu(), 2e-5, 1e-4)
+
+
 @pytest.mark.parametrize("epi", [ops.EPI_BIAS, ops.EPI_BIAS_GELU, ops.EPI_BIAS_RESIDUAL])
 @pytest.mark.parametrize("plan", [9, 14, 16, 21, 29])
 def test_gemm_write_through_launch_equals_plain(device, epi, plan):

@@ -10,23 +10,90 @@ static bool dtl_ok(const GemmPlan& p, int64_t k, int64_t lda, int64_t ldw, int e
   return k % (p.bkb / es) == 0 && (lda * es) % 16 == 0 && (ldw * es) % 16 == 0;
 }
 
-// Default tile choice.  For shapes the direct-to-LDS kernel takes, the
-// measured rule above; otherwise (odd K, misaligned rows) the staged plan
-// minimising (full-chip rounds of 256 workgroups) x (tile area / prior).
+// K-summation class of the default tile (plans of a class give the same
+// bits), by the shape alone; M counts in buckets of 64 rows, as the tile
+// timing of tjkernels/tiles.py (k_class) keys its shapes, so that a timed and
+// a default choice always agree in class.
+static int k_class(int64_t M, int64_t N, int64_t K) {
+  const int64_t m = (M + 63) / 64 * 64;
+  if ((m + 31) / 32 * ((N + 63) / 64) <= 256 && K >= 2048) return 4;
+  return (m + 127) / 128 * ((N + 63) / 64) <= 256 && K >= 512 ? 2 : 1;
+}
+
+// Estimated microseconds of a 2-byte launch on MI355X: with `tiles`
+// workgroups, `per_cu` of them resident per CU, a launch is `rounds` fillings
+// of the chip, in which the fullest CU runs `load` workgroups in all, each of
+// `steps` K tiles (per K group), and stores `mb` MB of output (read and
+// written, for a residual):
+//   c0 + c1 rounds + c2 rounds steps + c3 load + c4 load steps + c5 mb
+// (mb at 5 TB/s).  The coefficients are a non-negative least squares fit, by
+// relative error, over a sweep of 475 launches (16 to 16384 rows, widths 128 to
+// 8192, every epilogue) timed with every plan; each is within 4-11% on
+// average.  The tile the estimate picks is 0.7% slower than the best plan of
+// its class (geometric mean over the sweep); the fixed rule before it (8 from
+// two rounds of 256 x 256 tiles, 7 from 128 tiles of 128 x 128, else 9) was
+// 29% slower: 5430 x 3072 x 1024 47 us against 36, 128 x 512 x 2048 with the
+// residual 11.7 against 5.6.
+struct AutoTile {
+  int plan, per_cu;
+  float c[6];
+};
+static const AutoTile kAuto16[] = {
+    // one K group: 64 x 64, 96 x 128, 192 x 128, 128 x 128, 256 x 256, 192 x 384
+    {9, 5, {1.259f, 1.086f, 0.174f, 0.489f, 0.134f, 0.351f}},
+    {15, 2, {0.000f, 3.318f, 0.183f, 0.403f, 0.250f, 0.563f}},
+    {34, 2, {0.796f, 5.075f, 0.019f, 0.362f, 0.505f, 0.604f}},
+    {35, 2, {0.043f, 4.829f, 0.048f, 0.071f, 0.344f, 0.476f}},
+    {33, 1, {0.000f, 0.000f, 0.983f, 11.714f, 0.000f, 0.896f}},
+    {14, 1, {0.000f, 0.000f, 1.163f, 9.811f, 0.000f, 1.307f}},
+    // two K groups: 32 x 32, 32 x 64, 64 x 64, 128 x 64
+    {25, 2, {1.108f, 1.764f, 0.151f, 0.325f, 0.073f, 0.000f}},
+    {24, 1, {0.846f, 2.472f, 0.000f, 0.000f, 0.261f, 0.000f}},
+    {22, 1, {0.627f, 2.796f, 0.322f, 0.000f, 0.000f, 0.390f}},
+    {23, 1, {0.190f, 3.885f, 0.493f, 0.000f, 0.000f, 0.629f}},
+    // four K groups: 32 x 32, 32 x 64
+    {26, 1, {0.897f, 2.638f, 0.308f, 0.000f, 0.000f, 0.000f}},
+    {27, 1, {0.580f, 3.114f, 0.000f, 0.000f, 0.464f, 0.091f}},
+};
+
+static bool span_ok(const GemmPlan& p, int64_t lda, int64_t ldw, int es) {
+  return p.kind == kStaged || ((int64_t)p.bm * lda * es <= INT32_MAX && (int64_t)p.bn * ldw * es <= INT32_MAX);
+}
+
+// Default tile choice: for 2-byte types the least estimate among the tiles of
+// the shape's K class; for fp32 (and 2-byte rows too far apart for those
+// tiles' 31-bit offsets) the least (full-chip rounds of 256 workgroups) x
+// (tile area / prior).  The direct-to-LDS kernels take any K here: pieces of
+// the last K tile past K arrive as zeros.  (A plan asked for by id takes
+// whole K tiles only.)
 template <typename T>
-static int auto_plan(int64_t M, int64_t N, int64_t K, int64_t lda, int64_t ldw) {
+static int auto_plan(int64_t M, int64_t N, int64_t K, int64_t lda, int64_t ldw, int epi) {
   int count;
   const GemmPlan* p = plans<T>(&count);
-  if (sizeof(T) == 2 && dtl_ok(p[7], K, lda, ldw, sizeof(T))) {
-    // 256 x 256 tiles run one per CU: worth it when they come within 10% of
-    // whole rounds of the 256 CUs.  Measured (bf16): 8192 x 2048 x 8192 (one
-    // round) 193 us as plan 33, 216 as 8, 253 as 7; 8192 x 8192 x 2048 231 /
-    // 244 / 274; 5430 x 3072 x 1024 (264 tiles) 55 / 54 / 47.
-    const int64_t t256 = ((M + 255) / 256) * ((N + 255) / 256);
-    const int64_t t128 = ((M + 127) / 128) * ((N + 127) / 128);
-    if (10 * t256 >= 9 * 256 * ((t256 + 255) / 256)) return 33;
-    if (t128 >= 128) return 7;
-    return 9;
+  if constexpr (sizeof(T) == 2) {
+    // rows too far apart for the 128- (or, in small launches, 64-) row tiles'
+    // offsets are refused with whole K tiles, and staged otherwise
+    const int narrow = ((M + 127) / 128) * ((N + 127) / 128) >= 128 ? 7 : 9;
+    if (K % 64 == 0 && !span_ok(p[narrow], lda, ldw, sizeof(T))) return narrow;
+    const int cls = k_class(M, N, K);
+    const float mb = (float)M * (float)N * (epi_residual(epi) ? 8.f : 2.f) / 5e6f;
+    int best = -1;
+    float best_us = 0.f;
+    for (const AutoTile& t : kAuto16) {
+      const GemmPlan& q = p[t.plan];
+      if (q.ksplit != cls || !span_ok(q, lda, ldw, sizeof(T))) continue;
+      const int64_t tiles = ((M + q.bm - 1) / q.bm) * ((N + q.bn - 1) / q.bn), slots = 256 * t.per_cu;
+      const int64_t full = tiles / slots, rest = tiles % slots;
+      const float rounds = (float)(full + (rest > 0)), load = (float)(full * t.per_cu + (rest + 255) / 256);
+      const float steps = (float)((K + 63) / 64) / (float)cls;
+      const float us =
+          t.c[0] + rounds * (t.c[1] + t.c[2] * steps) + load * (t.c[3] + t.c[4] * steps) + t.c[5] * mb;
+      if (best < 0 || us < best_us) {
+        best = t.plan;
+        best_us = us;
+      }
+    }
+    if (best >= 0) return best;
   }
   int best = 0;
   double best_cost = 1e300;
@@ -50,11 +117,11 @@ static int gemm_checked(const void* a, int64_t lda, const void* w, int64_t ldw, 
   int count;
   const GemmPlan* p = plans<T>(&count);
   if (plan < -1 || plan >= count) return fail(TJK_EINVAL, "tjk_gemm_bias: plan %d out of range [-1,%d)", plan, count);
-  if (plan == -1) plan = auto_plan<T>(m, n, k, lda, ldw);
-  if (p[plan].kind != kStaged && !dtl_ok(p[plan], k, lda, ldw, sizeof(T)))
+  const bool by_rule = plan == -1;
+  if (by_rule) plan = auto_plan<T>(m, n, k, lda, ldw, epi);
+  if (!by_rule && p[plan].kind != kStaged && !dtl_ok(p[plan], k, lda, ldw, sizeof(T)))
     return fail(TJK_EUNSUPPORTED, "tjk_gemm_bias: plan %d needs k %% %d == 0", plan, (int)(p[plan].bkb / sizeof(T)));
-  if (p[plan].kind != kStaged && ((int64_t)p[plan].bm * lda * (int64_t)sizeof(T) > INT32_MAX ||
-                                  (int64_t)p[plan].bn * ldw * (int64_t)sizeof(T) > INT32_MAX))
+  if (!span_ok(p[plan], lda, ldw, sizeof(T)))
     return fail(TJK_EUNSUPPORTED, "tjk_gemm_bias: leading dimension too large for plan %d", plan);
   const GemmArgs g{a, lda, w, ldw, bias, c, ldc, (int)m, (int)n, (int)k, s, src};
   return run_gemm<T>(plan, epi, g);

@@ -177,7 +177,7 @@ __global__ __launch_bounds__(WM * WN * KSPLIT * 64) void gemm_dtl_kernel(
 
   f32x16 acc[FN][FM];
   zero_acc<T, FM, FN>(acc);
-  dtl_accumulate<T, BM, BN, WM, WN, BKB, STAGES, KSPLIT>(smem, A, lda, W, ldw, M, N, m0, n0, 0, K / G::BK, acc);
+  dtl_accumulate<T, BM, BN, WM, WN, BKB, STAGES, KSPLIT>(smem, A, lda, W, ldw, M, N, K, m0, n0, acc);
 
   constexpr int ACCF = FN * FM * 16;                   // accumulator floats per lane
   constexpr int XCH = (KSPLIT - 1) * NW * ACCF * 64 * 4;  // exchange bytes
@@ -257,7 +257,7 @@ __global__ __launch_bounds__((WM * WN + L) * 64) void gemm_ws_kernel(
   int pid_m, pid_n;
   tile_coords(blockIdx.x, (M + BM - 1) / BM, (N + BN - 1) / BN, pid_m, pid_n);
   const int m0 = pid_m * BM, n0 = pid_n * BN;
-  const int nk = K / G::BK;
+  const int nk = (K + G::BK - 1) / G::BK;
 
   if (wave >= NW) {
     // ------------------------------------------------------------ loaders
@@ -271,10 +271,15 @@ __global__ __launch_bounds__((WM * WN + L) * 64) void gemm_ws_kernel(
     // instruction q of loader lw fills rows (q L + lw) RPI .. +RPI-1 of the
     // stacked (A; W) tile; lane l lands at byte 16 l: row + l / CPR,
     // physical chunk l % CPR, so it fetches logical chunk (l % CPR) ^ swz(row)
+    // (the pieces of a last K tile past K point outside the range: zeros; L is
+    // even, so every instruction of a lane fetches the same chunk of its row)
+    static_assert(L % 2 == 0 && (BM / G::RPI) % 2 == 0, "row parity of the DMA instructions");
+    const uint32_t kend = (uint32_t)K * (uint32_t)sizeof(T);
+    const uint32_t lcb = (uint32_t)(((lane % G::CPR) ^ swz<BKB>(lw * G::RPI + lane / G::CPR)) << 4);
     auto dma = [&](int t, int q) {
       char* sb = smem + (t % STAGES) * STAGE;
       const int base = (q * L + lw) * G::RPI;  // wave-uniform
-      const uint32_t kb = (uint32_t)(t * BKB);
+      const uint32_t kb = (uint32_t)(t * BKB) + lcb < kend ? (uint32_t)(t * BKB) : (uint32_t)kPastEnd;
       if (base < BM) {
         const int r = base + lane / G::CPR;
         __builtin_amdgcn_raw_ptr_buffer_load_lds(

@@ -513,7 +513,7 @@ __device__ __forceinline__ void tile_coords(int bid, int tiles_m, int tiles_n, i
 // The DMA is issued on every iteration, past the end pointed outside the
 // buffer range (it moves nothing), which keeps the body one basic block;
 // scheduling directives interleave the MFMAs with the next step's ds_reads.
-// Requires K % (BKB / sizeof(T)) == 0 and 16-byte aligned rows.
+// Requires 16-byte aligned rows (K a multiple of 16 bytes).
 
 template <int BKB> __device__ __forceinline__ int swz(int r);
 template <> __device__ __forceinline__ int swz<128>(int r) { return (r & 7) ^ ((r >> 3) & 1); }
@@ -544,9 +544,10 @@ struct DtlGeom {
   static_assert(KS % 2 == 0, "fragment double buffer alternates per 16-deep step");
 };
 
-// acc += A[m0 : m0+BM, K tiles kt0..kt1) * W[n0 : n0+BN, same]^T for this
-// wave's sub-tile (K-split group kg takes K tiles kt0 + kg, kt0 + kg +
-// KSPLIT, ...).  On return every DMA has landed and the workgroup has met at
+// acc += A[m0 : m0+BM, :] * W[n0 : n0+BN, :]^T for this wave's sub-tile
+// (K-split group kg takes K tiles kg, kg + KSPLIT, ...; a last K tile that is
+// not whole has its 16-byte pieces past K pointed outside the buffer range,
+// so they arrive as zeros).  On return every DMA has landed and the workgroup has met at
 // a barrier, so the LDS ring may be reused.  (smem is deliberately not
 // __restrict__: with it the compiler stops telling the LDS DMA writes and
 // the fragment reads of different ring slots apart and waits for every DMA
@@ -554,7 +555,7 @@ struct DtlGeom {
 template <typename T, int BM, int BN, int WM, int WN, int BKB, int STAGES, int KSPLIT>
 __device__ __forceinline__ void dtl_accumulate(
     char* smem, const T* __restrict__ A, int64_t lda, const T* __restrict__ W, int64_t ldw,
-    int M, int N, int m0, int n0, int kt0, int kt1,
+    int M, int N, int K, int m0, int n0,
     f32x16 (&acc)[DtlGeom<T, BM, BN, WM, WN, BKB, STAGES, KSPLIT>::FN][DtlGeom<T, BM, BN, WM, WN, BKB, STAGES, KSPLIT>::FM]) {
   typedef DtlGeom<T, BM, BN, WM, WN, BKB, STAGES, KSPLIT> G;
   constexpr int NW = G::NW, KS = G::KS, CPR = G::CPR, RPI = G::RPI, CPS = G::CPS;
@@ -596,7 +597,15 @@ __device__ __forceinline__ void dtl_accumulate(
     const int r = (i * NW + wave) * RPI + lane / CPR;
     voff_w[i] = (uint32_t)(r * ldw * (int64_t)sizeof(T)) + (uint32_t)(((lane % CPR) ^ swz<BKB>(r)) << 4);
   }
-  const int nit = (kt1 - kt0 + KSPLIT - 1) / KSPLIT;  // ring steps per group
+  const int nkt = (K + G::BK - 1) / G::BK;
+  const int nit = (nkt + KSPLIT - 1) / KSPLIT;  // ring steps per group
+  // This lane's byte offset into the K tile.  A wave's instructions differ by
+  // NW rows of 8, so with an even NW swz's bit 3 of the row, and with it the
+  // chunk, is the same for all of them; with one wave it alternates.
+  const uint32_t kend = (uint32_t)K * (uint32_t)sizeof(T);
+  const uint32_t lcb = (uint32_t)(((lane % CPR) ^ swz<BKB>(wave * RPI + lane / CPR)) << 4);
+  static_assert(NW == 1 || (NW % 2 == 0 && (BM / RPI) % 2 == 0), "row parity of the DMA instructions");
+  static_assert(BKB == 128, "swizzle of 128-byte rows");
   // Eight-wave tiles with 96 x 96 (or larger) wave tiles issue every DMA
   // instruction from waves 0-3 (one per SIMD), twice their share, and none
   // from waves 4-7: a wave whose DMA cannot issue yet stalls its own in-order
@@ -611,12 +620,14 @@ __device__ __forceinline__ void dtl_accumulate(
   constexpr int NDW = ASYM ? 2 * NDMA : NDMA;  // DMA instructions per issuing wave per tile
   const bool issuer = !ASYM || wave < NW / 2;
   // DMA instruction q (q < DA: A rows, else W rows) of this group's step it
-  // into its slot; past the segment it points outside the range and moves
-  // nothing.
+  // into its slot; past K it points outside the range and moves nothing.
+  auto k_off = [&](int it, int i) __attribute__((always_inline)) {
+    const uint32_t kt = (uint32_t)((it * KSPLIT + kg) * BKB);
+    return kt + (NW == 1 && (i & 1) ? lcb ^ 16u : lcb) < kend ? kt : (uint32_t)kPastEnd;
+  };
   auto dma1 = [&](int it, int q) {
     char* sb = gsm + (it % STAGES) * STAGE;
-    const int kt = kt0 + it * KSPLIT + kg;
-    const uint32_t kb = kt < kt1 ? (uint32_t)(kt * BKB) : (uint32_t)kPastEnd;
+    const uint32_t kb = k_off(it, q < DA ? q : q - DA);
     if (q < DA)
       __builtin_amdgcn_raw_ptr_buffer_load_lds(rsa, (lds_void*)(sb + (q * NW + wave) * 1024), 16,
                                                (uint32_t)(voff_a[q] + kb), 0, 0, 0);
@@ -628,8 +639,7 @@ __device__ __forceinline__ void dtl_accumulate(
   // (q' NW/2 + w) RPI .. +RPI-1 of the stacked (A; W) tile, q' < 2 NDMA
   auto dma2 = [&](int it, int q2) {
     char* sb = gsm + (it % STAGES) * STAGE;
-    const int kt = kt0 + it * KSPLIT + kg;
-    const uint32_t kb = kt < kt1 ? (uint32_t)(kt * BKB) : (uint32_t)kPastEnd;
+    const uint32_t kb = k_off(it, 0);
     const int base = (q2 * (NW / 2) + wave) * RPI;  // wave-uniform
     if (base < BM) {
       const int r = base + lane / CPR;
