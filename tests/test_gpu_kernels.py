@@ -549,11 +549,49 @@ def _attn_ref(qkv, causal, key_mask=None):
     q, k, v = (qkv[:, :, i].transpose(1, 2).double() for i in range(3))
     scores = (q @ k.transpose(-2, -1)) * hd ** -0.5
     if causal:
-        scores = scores.masked_fill(torch.ones(s, s, dtype=torch.bool).triu(1), float("-inf"))
+        scores = scores.masked_fill(torch.ones(s, s, dtype=torch.bool, device=qkv.device).triu(1), float("-inf"))
     if key_mask is not None:
         scores = scores.masked_fill(~key_mask[:, None, None, :], float("-inf"))
     probs = torch.softmax(scores, -1).nan_to_num(0.0)
     return (probs @ v).transpose(1, 2).reshape(b * s, h * hd)
+
+
+@pytest.mark.parametrize("causal", [True, False])
+@pytest.mark.parametrize("hd", [64, 128])
+@pytest.mark.parametrize("dt,seq,heads", [(torch.bfloat16, 129, 2), (torch.float16, 256, 1), (torch.bfloat16, 515, 2),
+                                          (torch.float16, 8064, 1), (torch.bfloat16, 8065, 1)])
+def test_flash_masked_lists_keys(device, dt, seq, heads, hd, causal):
+    """Masked plan 0 over the admissible keys only (head_dim 64 / 128, up to
+    8064 keys; one more runs the kernel that masks tiles): every key, none,
+    a quarter missing, one at either end, whole 64-key blocks missing, exactly
+    64 and 65 keys; and with prefix lengths on top.  K of the masked keys is
+    NaN: only the admissible keys may enter."""
+    g = _gen(seq + hd)
+    keep = torch.rand(8, seq, generator=g) < 0.75
+    keep[0], keep[1] = True, False
+    keep[2], keep[2, 0] = False, True
+    keep[3], keep[3, -1] = False, True
+    keep[4, 64:192] = False
+    keep[5], keep[5, 30:94] = False, True
+    keep[6], keep[6, 30:95] = False, True
+    if seq > 1000:
+        keep = keep[[1, 4, 7]]
+    b = keep.shape[0]
+    lengths = torch.randint(0, seq + 1, (b,), generator=g).int()
+    qkv = torch.randn(b, seq, 3, heads, hd, generator=g).to(dt)
+    qkv[:, :, 1][~keep] = float("nan")
+    for lens in (None, lengths):
+        if lens is not None and seq > 1000:
+            continue
+        mask = keep if lens is None else keep & (torch.arange(seq)[None, :] < lens[:, None])
+        clean = qkv.clone()
+        clean[:, :, 1][~keep] = 0
+        ref = _attn_ref(clean.to(device), causal, mask.to(device)).cpu()
+        out = torch.full((b * seq, heads * hd), float("nan"), dtype=dt, device=device)
+        ops.flash_attention(qkv.to(device), out, causal=causal, key_mask=keep.to(device),
+                            lengths=None if lens is None else lens.to(device), plan=0)
+        torch.cuda.synchronize()
+        _close(out, ref, OUT_RTOL[dt], 4e-3 if dt == torch.bfloat16 else 1e-3)
 
 
 @pytest.mark.parametrize("dt", [torch.bfloat16, torch.float16, torch.float32])

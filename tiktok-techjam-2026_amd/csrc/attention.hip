@@ -536,6 +536,10 @@ __global__ __launch_bounds__(64) void flash_short_kernel(
 constexpr int kFaSc1 = 16, kFaSc0Sc1 = 17;
 typedef __attribute__((address_space(3))) void lds_void;
 
+// Most keys a masked launch of the DMA ring can list (16 KB beside the 64 KB
+// ring of head_dim 64, two workgroups per CU).
+constexpr int kFaListKeys = 8064;
+
 constexpr int kFaSpinLimit = 1 << 20;  // polls of a split item's flag before giving up (>= 0.1 s)
 
 // Buffer descriptor over `bytes` bytes at p (stride 0, raw dword access).
@@ -579,25 +583,39 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(HDP <= 
   constexpr int KPT = KITEMS / NT, VPT = (VITEMS + NT - 1) / NT;
   static_assert(KITEMS % NT == 0, "K tile must split evenly over the threads");
 
-  // K / V ring.  DMA (head_dim 64 / 128 with the full head dimension, no
-  // key mask): tiles are copied straight into LDS by buffer_load ... lds, K
+  // K / V ring.  DMA (head_dim 64 / 128 with the full head dimension): tiles
+  // are copied straight into LDS by buffer_load ... lds, K
   // and V both key-major with 128- / 256-byte rows whose 16-byte chunks are
   // XOR-swizzled by row, and V^T fragments are gathered with the transposing
   // ds_read_b64_tr_b16.  Otherwise tiles pass through registers, V stored
   // transposed.
-  constexpr bool DMA = FULLHD && !KEYMASK && HDP >= 64;
+  constexpr bool DMA = FULLHD && HDP >= 64;
+  // LIST (DMA ring with a key mask): the workgroup lists its admissible keys
+  // first and the ring's tiles hold those keys only, 64 of them each, so the
+  // tiles need no mask bytes, run the interior loop up to the diagonal, and
+  // masked keys cost nothing.  Key limits (kend, lim, ...) then count listed
+  // keys.  Before, every tile of a masked launch loaded 32 mask bytes per lane
+  // and ran the unpipelined loop.  Measured with a quarter of the keys masked:
+  // 8 x 512 x 12 heads of 64, fp16, 27.6 -> 16.4 us (14.0 without a mask); 4 x
+  // 2048 x 16 heads of 64, bf16 causal, 109 (plan 1) -> 48 us (47); 2 x 4096 x
+  // 16 heads of 128, causal, 406 -> 114 us (137).
+  constexpr bool LIST = DMA && KEYMASK;
   constexpr int RB = HDP * (int)sizeof(T);  // DMA: bytes per K / V row
   constexpr int CPR = RB / 16, RPI = 64 / CPR, TILE_B = BNK * RB;
   char* smem;  // DMA ring: slot st holds K at st * 2 TILE_B, V TILE_B later
   T (*sK)[BNK * LDK];
   T (*sV)[HDP * LDV];
   int* s_flag;  // the split-item merge's published flag
+  uint16_t* s_list = nullptr;  // LIST: the listed keys
   if constexpr (DMA) {
-    __shared__ __attribute__((aligned(1024))) char ring[NST * 2 * TILE_B + 16];
+    // (one array: LDS copies and reads of separate arrays would be ordered
+    // against each other by the compiler)
+    __shared__ __attribute__((aligned(1024))) char ring[NST * 2 * TILE_B + 16 + (LIST ? 2 * kFaListKeys : 0)];
     smem = ring;
     sK = nullptr;
     sV = nullptr;
     s_flag = reinterpret_cast<int*>(ring + NST * 2 * TILE_B);
+    s_list = reinterpret_cast<uint16_t*>(ring + NST * 2 * TILE_B + 16);
   } else {
     __shared__ __attribute__((aligned(16))) T k_ring[NST][BNK * LDK];
     __shared__ __attribute__((aligned(16))) T v_ring[NST][HDP * LDV];
@@ -637,6 +655,63 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(HDP <= 
   if (q0 >= Sb) return;  // the whole workgroup: past this sequence's end
   int kend = causal ? min(q0 + BMQ, Sb) : Sb;
   kend = min(kend, kv_len);
+  // Key limits: lane's query admits keys below lim, the wave's first and last
+  // query below lim_lo and lim_hi, the workgroup's first below lim_wg.
+  int lim = 0, lim_lo = wq0 + 1, lim_hi = wq0 + 32, lim_wg = q0;
+  if constexpr (LIST) {
+    // Admissible keys in order, 64 at a time: each wave ballots every NW-th
+    // block of 64 mask bytes, the counts are summed over the blocks (lane l:
+    // blocks 2 l and 2 l + 1), and each block's keys go to the list at its
+    // sum.  The ballots and sums lie in the ring's last slot, which the first
+    // copies do not touch.
+    uint64_t* const bits = reinterpret_cast<uint64_t*>(smem + (NST - 1) * 2 * TILE_B);
+    int* const sums = reinterpret_cast<int*>(bits + 128);
+    const int nblk = (kend + 63) / 64;
+    const uint8_t* const km = key_mask + (int64_t)b * S;
+    for (int j0 = wave; j0 < 128; j0 += 8 * NW) {
+      uint8_t v[8];  // eight blocks' bytes in flight together
+#pragma unroll
+      for (int u = 0; u < 8; ++u) v[u] = j0 < nblk ? km[min((j0 + u * NW) * 64 + lane, S - 1)] : 0;
+#pragma unroll
+      for (int u = 0; u < 8; ++u) {
+        const uint64_t m = __ballot((j0 + u * NW) * 64 + lane < kend && v[u] != 0);
+        if (lane == 0) bits[j0 + u * NW] = m;
+      }
+    }
+    __syncthreads();
+    const int c0 = __popcll(bits[2 * lane]), c1 = __popcll(bits[2 * lane + 1]);
+    int sum = c0 + c1;
+#pragma unroll
+    for (int d = 1; d < 64; d <<= 1) {
+      const int up = __shfl_up(sum, d);
+      sum += lane >= d ? up : 0;
+    }
+    if (wave == 0) {
+      sums[2 * lane] = sum - c0 - c1;
+      sums[2 * lane + 1] = sum - c1;
+    }
+    const int listed = __builtin_amdgcn_readlane(sum, 63);
+    __syncthreads();
+    for (int j = wave; j < nblk; j += NW) {
+      const uint64_t m = bits[j];
+      const int at = sums[j] + __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0));
+      if (m >> lane & 1) s_list[at] = (uint16_t)(j * 64 + lane);
+    }
+    // listed keys up to key q
+    auto upto = [&](int q) __attribute__((always_inline)) {
+      const int c = max(min(q, kend - 1), 0);
+      return sums[c >> 6] + __popcll(bits[c >> 6] & (~0ull >> (63 - (c & 63))));
+    };
+    lim = lim_lo = lim_hi = lim_wg = listed;
+    if (causal && kend > 0) {
+      lim = upto(wq0 + l32);
+      lim_lo = __builtin_amdgcn_readlane(lim, 0);
+      lim_hi = __builtin_amdgcn_readlane(lim, 31);
+      lim_wg = __builtin_amdgcn_readfirstlane(upto(q0));
+    }
+    kend = listed;
+    __syncthreads();
+  }
   const int nkt = (kend + BNK - 1) / BNK;
   t_hi = min(t_hi, nkt);
 
@@ -742,9 +817,34 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(HDP <= 
     const int r = (q * NW + wave) * RPI + lane / CPR;
     dvoff[q] = (uint32_t)r * row_bytes + (uint32_t)(((lane % CPR) ^ swz(r)) << 4);
   }
+  // LIST: this lane's listed key of each DMA instruction of the tile that is
+  // copied next, read from the list one tile ahead
+  int dkey[LIST ? NDK : 1];
+  auto next_keys = [&](int t) __attribute__((always_inline)) {
+#pragma unroll
+    for (int q = 0; q < (LIST ? NDK : 0); ++q)
+      dkey[q] = s_list[min(t * BNK + (q * NW + wave) * RPI + lane / CPR, kFaListKeys - 1)];
+  };
   // K and V of key tile t into ring slot st (a tile past the item's range
   // gets an empty descriptor and moves nothing)
   auto dma_kv = [&](int t, int st) __attribute__((always_inline)) {
+    if constexpr (LIST) {
+      const u32x4 rk = fa_rsrc(qbase + sc, span), rv = fa_rsrc(qbase + 2 * sc, span);
+      const uint32_t kb = lds_ring + (uint32_t)(st * 2 * TILE_B + wave * 1024);
+      uint32_t off[NDK];
+#pragma unroll
+      for (int q = 0; q < NDK; ++q) {
+        const int r = (q * NW + wave) * RPI + lane / CPR;
+        off[q] = t * BNK + r < kend ? (uint32_t)dkey[q] * row_bytes + (uint32_t)(((lane % CPR) ^ swz(r)) << 4)
+                                    : 0x80000000u;  // past the list, and any range: zeros
+      }
+#pragma unroll
+      for (int q = 0; q < NDK; ++q) fa_lds_dma16(rk, off[q], kb + q * NW * 1024);
+#pragma unroll
+      for (int q = 0; q < NDK; ++q) fa_lds_dma16(rv, off[q], kb + TILE_B + q * NW * 1024);
+      next_keys(t + 1);
+      return;
+    }
     const int64_t t_elems = (int64_t)t * BNK * ss;
     const int nrec = t < t_hi ? span - (int)(t_elems * (int64_t)sizeof(T)) : 0;
     const u32x4 rsk = fa_rsrc(qbase + sc + t_elems, nrec), rsv = fa_rsrc(qbase + 2 * sc + t_elems, nrec);
@@ -887,6 +987,14 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(HDP <= 
   // register r of block kb is key k0 + kb*32 + 16*(r/8) + 8*hi + r%8
   auto mask_tile = [&](int t, f32x16 (&sa)[2]) {
     const int k0 = t * BNK, q = wq0 + l32;
+    if constexpr (LIST) {
+#pragma unroll
+      for (int kb = 0; kb < 2; ++kb)
+#pragma unroll
+        for (int r = 0; r < 16; ++r)
+          sa[kb][r] = k0 + kb * 32 + 16 * (r >> 3) + 8 * hi + (r & 7) < lim ? sa[kb][r] : -INFINITY;
+      return;
+    }
     const int lim = causal ? min(q + 1, kend) : kend;
     // mask bytes all loaded before any is used (see flash_fwd_kernel)
     uint8_t km[2][16];
@@ -1055,6 +1163,7 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(HDP <= 
   if constexpr (DMA) {
     // the first three tiles in flight at once; the first two have landed
     // at the barrier
+    next_keys(t_lo);
     dma_kv(t_lo, 0);
     dma_kv(t_lo + 1, 1);
     dma_kv(t_lo + 2, 2);
@@ -1080,7 +1189,7 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(HDP <= 
   if (t_hi > t_lo) qk(0, scur);
   // Interior tiles: every key below the workgroup's first query and inside
   // the sequence, and a next tile exists in this item's range.
-  int n_int = KEYMASK ? 0 : min(causal ? q0 / BNK : nkt, min(kend / BNK, t_hi - 1));
+  int n_int = KEYMASK && !LIST ? 0 : min(causal ? lim_wg / BNK : nkt, min(kend / BNK, t_hi - 1));
   n_int = max(n_int, t_lo);
   int t = t_lo;
   // an unmasked first tile starts the offset at its row max, so the
@@ -1134,13 +1243,13 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(HDP <= 
       load_kv(t + 3);
     }
     f32x16 snext[2];
-    const bool act_next = t + 1 < t_hi && (!causal || (t + 1) * BNK <= wq0 + 31);
+    const bool act_next = t + 1 < t_hi && (!causal || (t + 1) * BNK < lim_hi);
     if (act_next) qk(slot_of(t + 1), snext);
-    const bool act = !causal || t * BNK <= wq0 + 31;
+    const bool act = !causal || t * BNK < lim_hi;
     if (act) {
       // a tile below the wave's first query and inside the sequence (the
       // first diagonal tile for the upper waves) needs no mask
-      if (KEYMASK || (causal && t * BNK + BNK - 1 > wq0) || t * BNK + BNK > kend) mask_tile(t, scur);
+      if ((KEYMASK && !LIST) || (causal && t * BNK + BNK > lim_lo) || t * BNK + BNK > kend) mask_tile(t, scur);
       softmax_pv(slot_of(t), scur);
     }
     step_barrier();
@@ -1375,15 +1484,20 @@ static int launch_sched(const void* qkv, int64_t ss, int64_t sc, int64_t sh, voi
   return check_launch("tjk_flash_fwd_sched");
 }
 
+// Whether a masked launch of plan 0 lists its admissible keys.
+static bool flash_lists(int hd, int S) { return (hd == 64 || hd == 128) && S <= kFaListKeys; }
+
 template <typename T, int HDP>
 static int launch_pipe(const void* qkv, int64_t sb, int64_t ss, int64_t sc, int64_t sh, void* out,
                        int64_t ld_out, int B, int S, int H, int hd, float scale_log2, int causal,
                        const int32_t* lengths, const uint8_t* key_mask, const int32_t* cu_seqlens,
                        hipStream_t st) {
-  // head_dim 128 without a key mask: 8 waves and 256 queries per workgroup
-  // (see flash_pipe_kernel; with a key mask that variant would spill)
+  // head_dim 128: 8 waves and 256 queries per workgroup (see
+  // flash_pipe_kernel), except for masked launches that do not list their keys
+  // (that variant would spill)
   constexpr int NW8 = HDP == 128 ? 8 : 4;
-  const int nw = key_mask == nullptr ? NW8 : 4;
+  const bool list = key_mask != nullptr && flash_lists(hd, S);
+  const int nw = key_mask == nullptr || list ? NW8 : 4;
   const int nqb = (S + 32 * nw - 1) / (32 * nw);
   const int64_t nblk = (int64_t)nqb * B * H;
   if (nblk > INT32_MAX) return fail(TJK_EUNSUPPORTED, "tjk_flash_fwd: grid too large");
@@ -1399,7 +1513,11 @@ static int launch_pipe(const void* qkv, int64_t sb, int64_t ss, int64_t sc, int6
                      (const T*)qkv, sb, ss, sc, sh, (T*)out, ld_out, B, S, H, hd, scale_log2, causal, lengths,  \
                      key_mask, cu_seqlens, nqb, (const int4*)nullptr, 0, (float*)nullptr, (int*)nullptr, 0, grp)
   if (key_mask != nullptr) {
-    if (hd == HDP) TJK_PIPE(true, true, 4); else TJK_PIPE(true, false, 4);
+    if constexpr (HDP >= 64) {
+      if (list) TJK_PIPE(true, true, NW8); else TJK_PIPE(true, false, 4);
+    } else {
+      TJK_PIPE(true, false, 4);
+    }
   } else {
     if (hd == HDP) TJK_PIPE(false, true, NW8); else TJK_PIPE(false, false, NW8);
   }
@@ -1535,7 +1653,8 @@ extern "C" int tjk_flash_fwd(const void* qkv, int64_t stride_b, int64_t stride_s
   // at hd 128 too since its 8-wave workgroups (causal 16 x 512: 50.5 vs
   // 53.0 us, 4 x 2048: 95.1 vs 122.6 us, 2 x 8192: 615 vs 743 us); plans 2
   // and 3 were slower on every BASELINE shape.
-  // With a key mask plan 0 runs every tile through its masked
+  // With a key mask plan 0 lists the admissible keys where it can (see
+  // flash_pipe_kernel); otherwise it runs every tile through its masked
   // (unpipelined) loop: plan 1 from S = 2048 (padded C4 with a per-key
   // mask: 129 vs 168 us).  A sequence of one 128-query block has only
   // diagonal tiles and nothing to pipeline: plan 1 there too (C2's
@@ -1547,7 +1666,7 @@ extern "C" int tjk_flash_fwd(const void* qkv, int64_t stride_b, int64_t stride_s
     if (seq <= 128)
       plan_id = 4;
     else
-      plan_id = (pipe_ok && (key_mask == nullptr || seq < 2048)) ? 0 : 1;
+      plan_id = (pipe_ok && (key_mask == nullptr || flash_lists(head_dim, seq) || seq < 2048)) ? 0 : 1;
   }
   if (plan_id == 0 && !pipe_ok) plan_id = 1;
   const float scale_log2 = scale * 1.4426950408889634f;
