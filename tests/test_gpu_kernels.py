@@ -239,6 +239,18 @@ def test_gemm_default_tile_takes_any_k(device, dt, m, n, k):
     _close(res, (ref + r0.to(device).double()).cpu(), 2e-5, 1e-4)
 
 
+@pytest.mark.parametrize("m,n,k", [  # K past whole 32-deep tiles; the tile the default rule takes:
+    (1, 4, 4), (700, 1028, 200),         # 64 x 64
+    (130, 68, 260), (33, 1000, 2052),    # 32 x 32, K split in 4
+    (700, 1024, 2052),                   # the last tile count that splits
+    (2050, 3068, 772),                   # 128 x 64
+    (4100, 4092, 68),                    # 128 x 128
+])
+def test_gemm_default_tile_fp32(device, m, n, k):
+    for epi in (ops.EPI_BIAS, ops.EPI_BIAS_GELU, ops.EPI_BIAS_RESIDUAL):
+        _gemm_case(device, m, n, k, torch.float32, epi, -1)
+
+
 @pytest.mark.parametrize("epi", [ops.EPI_BIAS, ops.EPI_BIAS_GELU, ops.EPI_BIAS_RESIDUAL])
 @pytest.mark.parametrize("plan", [9, 14, 16, 21, 29])
 def test_gemm_write_through_launch_equals_plain(device, epi, plan):
@@ -554,6 +566,34 @@ def _attn_ref(qkv, causal, key_mask=None):
         scores = scores.masked_fill(~key_mask[:, None, None, :], float("-inf"))
     probs = torch.softmax(scores, -1).nan_to_num(0.0)
     return (probs @ v).transpose(1, 2).reshape(b * s, h * hd)
+
+
+@pytest.mark.parametrize("causal", [True, False])
+@pytest.mark.parametrize("hd", [24, 64])
+@pytest.mark.parametrize("batch,seq,heads", [(2, 129, 2), (1, 192, 3), (2, 515, 2), (22, 260, 4)])
+def test_flash_fp32_default_plan(device, batch, seq, heads, hd, causal):
+    """fp32 without a plan: 64-query workgroups with two key splits (few
+    blocks) and, at 22 x 260 x 4, the 128-query plans; padded, with a key
+    mask, with lengths, and packed."""
+    g = _gen(seq + hd)
+    qkv = torch.randn(batch, seq, 3, heads, hd, generator=g)
+    keep = torch.rand(batch, seq, generator=g) < 0.7
+    keep[0, :] = False
+    keep[-1, :100] = False
+    lens = torch.randint(0, seq + 1, (batch,), generator=g).int()
+    short = torch.arange(seq)[None, :] < lens[:, None]
+    for mask, kw in ((None, {}), (keep, dict(key_mask=keep.to(device))), (short, dict(lengths=lens.to(device)))):
+        out = torch.full((batch * seq, heads * hd), float("nan"), device=device)
+        ops.flash_attention(qkv.to(device), out, causal=causal, **kw)
+        torch.cuda.synchronize()
+        _close(out, _attn_ref(qkv, causal, mask), OUT_RTOL[torch.float32], 1e-5)
+    rows = torch.cat([qkv[b, :n] for b, n in enumerate(lens.tolist())])
+    cu = torch.tensor([0] + lens.cumsum(0).tolist(), dtype=torch.int32, device=device)
+    out = torch.full((rows.shape[0], heads * hd), float("nan"), device=device)
+    ops.flash_attention(rows.to(device), out, causal=causal, cu_seqlens=cu, max_seqlen=seq)
+    torch.cuda.synchronize()
+    ref = torch.cat([_attn_ref(qkv[b:b + 1, :n], causal) for b, n in enumerate(lens.tolist())])
+    _close(out, ref, OUT_RTOL[torch.float32], 1e-5)
 
 
 @pytest.mark.parametrize("causal", [True, False])

@@ -14,13 +14,20 @@ static bool dtl_ok(const GemmPlan& p, int64_t k, int64_t lda, int64_t ldw, int e
 // bits), by the shape alone; M counts in buckets of 64 rows, as the tile
 // timing of tjkernels/tiles.py (k_class) keys its shapes, so that a timed and
 // a default choice always agree in class.
+template <typename T>
 static int k_class(int64_t M, int64_t N, int64_t K) {
   const int64_t m = (M + 63) / 64 * 64;
+  if (sizeof(T) == 4) {
+    // at 128 tiles of 64 x 64 the split is 1.2-1.8 times as fast, at 192 with
+    // K >= 2048 1.2; at 192 with less K, and at 256, it is slower
+    const int64_t tiles = m / 64 * ((N + 63) / 64);
+    return (tiles <= 128 && K >= 256) || (tiles <= 192 && K >= 2048) ? 4 : 1;
+  }
   if ((m + 31) / 32 * ((N + 63) / 64) <= 256 && K >= 2048) return 4;
   return (m + 127) / 128 * ((N + 63) / 64) <= 256 && K >= 512 ? 2 : 1;
 }
 
-// Estimated microseconds of a 2-byte launch on MI355X: with `tiles`
+// Estimated microseconds of a launch on MI355X: with `tiles`
 // workgroups, `per_cu` of them resident per CU, a launch is `rounds` fillings
 // of the chip, in which the fullest CU runs `load` workgroups in all, each of
 // `steps` K tiles (per K group), and stores `mb` MB of output (read and
@@ -33,7 +40,10 @@ static int k_class(int64_t M, int64_t N, int64_t K) {
 // its class (geometric mean over the sweep); the fixed rule before it (8 from
 // two rounds of 256 x 256 tiles, 7 from 128 tiles of 128 x 128, else 9) was
 // 29% slower: 5430 x 3072 x 1024 47 us against 36, 128 x 512 x 2048 with the
-// residual 11.7 against 5.6.
+// residual 11.7 against 5.6.  fp32: 208 launches, each coefficient set within
+// 1.3-2.5% on average; 0.6% slower than the best plan, where the rule before
+// it (rounds x area / prior) was 58% slower (1284 x 1536 x 512 37 us against
+// 22.6, 128 x 512 x 512 12.6 against 6.4).
 struct AutoTile {
   int plan, per_cu;
   float c[6];
@@ -56,44 +66,59 @@ static const AutoTile kAuto16[] = {
     {27, 1, {0.580f, 3.114f, 0.000f, 0.000f, 0.464f, 0.091f}},
 };
 
+static const AutoTile kAuto32[] = {
+    // 128 x 128, 64 x 64, 128 x 64; the one tile with four K groups
+    {2, 2, {3.105f, 0.670f, 0.234f, 1.139f, 1.709f, 0.626f}},
+    {4, 5, {2.625f, 0.000f, 0.169f, 0.000f, 0.469f, 1.167f}},
+    {6, 3, {3.423f, 0.000f, 0.204f, 0.000f, 0.874f, 1.150f}},
+    {5, 2, {}},
+};
+
 static bool span_ok(const GemmPlan& p, int64_t lda, int64_t ldw, int es) {
   return p.kind == kStaged || ((int64_t)p.bm * lda * es <= INT32_MAX && (int64_t)p.bn * ldw * es <= INT32_MAX);
 }
 
-// Default tile choice: for 2-byte types the least estimate among the tiles of
-// the shape's K class; for fp32 (and 2-byte rows too far apart for those
-// tiles' 31-bit offsets) the least (full-chip rounds of 256 workgroups) x
-// (tile area / prior).  The direct-to-LDS kernels take any K here: pieces of
-// the last K tile past K arrive as zeros.  (A plan asked for by id takes
-// whole K tiles only.)
+// The tile of `table` with the least estimate in the shape's K class, or -1.
+template <typename T, int NT>
+static int least_estimate(const AutoTile (&table)[NT], const GemmPlan* p, int64_t M, int64_t N, int64_t K, int64_t lda,
+                          int64_t ldw, int epi) {
+  constexpr int BK = 128 / sizeof(T);
+  const int cls = k_class<T>(M, N, K);
+  const float mb = (float)M * (float)N * (epi_residual(epi) ? 8.f : (float)sizeof(T)) / 5e6f;
+  const float steps = (float)((K + BK - 1) / BK) / (float)cls;
+  int best = -1;
+  float best_us = 0.f;
+  for (const AutoTile& t : table) {
+    const GemmPlan& q = p[t.plan];
+    if (q.ksplit != cls || !span_ok(q, lda, ldw, sizeof(T))) continue;
+    const int64_t tiles = ((M + q.bm - 1) / q.bm) * ((N + q.bn - 1) / q.bn), slots = 256 * t.per_cu;
+    const int64_t full = tiles / slots, rest = tiles % slots;
+    const float rounds = (float)(full + (rest > 0)), load = (float)(full * t.per_cu + (rest + 255) / 256);
+    const float us = t.c[0] + rounds * (t.c[1] + t.c[2] * steps) + load * (t.c[3] + t.c[4] * steps) + t.c[5] * mb;
+    if (best < 0 || us < best_us) {
+      best = t.plan;
+      best_us = us;
+    }
+  }
+  return best;
+}
+
+// Default tile choice: the least estimate.  The direct-to-LDS kernels take
+// any K here: pieces of the last K tile past K arrive as zeros.  (A plan asked
+// for by id takes whole K tiles only.)  Rows too far apart for those tiles'
+// 31-bit offsets go by the least (full-chip rounds of 256 workgroups) x (tile
+// area / prior) over the plans that take the K: staged, or refused.
 template <typename T>
 static int auto_plan(int64_t M, int64_t N, int64_t K, int64_t lda, int64_t ldw, int epi) {
   int count;
   const GemmPlan* p = plans<T>(&count);
   if constexpr (sizeof(T) == 2) {
-    // rows too far apart for the 128- (or, in small launches, 64-) row tiles'
-    // offsets are refused with whole K tiles, and staged otherwise
     const int narrow = ((M + 127) / 128) * ((N + 127) / 128) >= 128 ? 7 : 9;
     if (K % 64 == 0 && !span_ok(p[narrow], lda, ldw, sizeof(T))) return narrow;
-    const int cls = k_class(M, N, K);
-    const float mb = (float)M * (float)N * (epi_residual(epi) ? 8.f : 2.f) / 5e6f;
-    int best = -1;
-    float best_us = 0.f;
-    for (const AutoTile& t : kAuto16) {
-      const GemmPlan& q = p[t.plan];
-      if (q.ksplit != cls || !span_ok(q, lda, ldw, sizeof(T))) continue;
-      const int64_t tiles = ((M + q.bm - 1) / q.bm) * ((N + q.bn - 1) / q.bn), slots = 256 * t.per_cu;
-      const int64_t full = tiles / slots, rest = tiles % slots;
-      const float rounds = (float)(full + (rest > 0)), load = (float)(full * t.per_cu + (rest + 255) / 256);
-      const float steps = (float)((K + 63) / 64) / (float)cls;
-      const float us =
-          t.c[0] + rounds * (t.c[1] + t.c[2] * steps) + load * (t.c[3] + t.c[4] * steps) + t.c[5] * mb;
-      if (best < 0 || us < best_us) {
-        best = t.plan;
-        best_us = us;
-      }
-    }
+    const int best = least_estimate<T>(kAuto16, p, M, N, K, lda, ldw, epi);
     if (best >= 0) return best;
+  } else if (span_ok(p[3], lda, ldw, sizeof(T))) {
+    return least_estimate<T>(kAuto32, p, M, N, K, lda, ldw, epi);
   }
   int best = 0;
   double best_cost = 1e300;

@@ -535,6 +535,8 @@ int run_gemm(int plan, int epi, const GemmArgs& g) {
       TJK_GEMM_CASE(2, D2, 128, 128, 2, 2)
       TJK_GEMM_CASE(3, D2, 256, 128, 2, 2)
       TJK_GEMM_CASE(4, D2, 64, 64, 2, 2)
+      TJK_GEMM_CASE(5, D2K4, 32, 32, 1, 1)
+      TJK_GEMM_CASE(6, D2, 128, 64, 2, 2)
     }
   } else {
     switch (plan) {

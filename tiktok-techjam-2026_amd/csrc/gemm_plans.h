@@ -96,6 +96,11 @@ static const GemmPlan kPlans32[] = {
     {kDtl, 128, 128, 2, 2, 128, 2, 1.0},     // 2
     {kDtl, 256, 128, 2, 2, 128, 2, 1.0},     // 3
     {kDtl, 64, 64, 2, 2, 128, 2, 0.5},       // 4
+    // 5: K split between four one-wave groups, for launches whose 64 x 64 tiles
+    // leave most CUs idle (256 x 1024 x 1024 22.9 -> 9.4 us); 6: the tile
+    // between 64 x 64 and 128 x 128 (5690 x 1024 x 1792 180 -> 168 us).
+    {kDtl, 32, 32, 1, 1, 128, 2, 0.3, 4},    // 5 4 waves, 64 KB
+    {kDtl, 128, 64, 2, 2, 128, 2, 0.6},      // 6 wave tile 64x32
 };
 
 template <typename T>

@@ -24,7 +24,10 @@ whatever the timing picks.  ``k_class`` chooses the K split when a launch of
 split to shorten the serial chain of K tiles (the launch-bound projections
 of C2 and C3's FFN2: 10.6 -> 8.5 us and 26.1 -> 23.0 us measured on MI355X),
 and the four-way split when one round of 32 x 64 tiles covers the launch and
-K >= 2048 (C2's FFN2).
+K >= 2048 (C2's FFN2).  In fp32 the four-way split takes launches of up to 128
+tiles of 64 x 64 (192 with K >= 2048), else class 1.  The library's own rule
+(k_class in csrc/gemm.hip) is the same, so a launch without a plan keeps these
+classes too.
 
 The LayerNorm-prologue GEMM (``tjk_gemm_ln``, LayerNorm computed inside
 the GEMM for launch-bound row counts) has its own plans, 32-row tiles of
@@ -66,7 +69,8 @@ from . import _lib, ops, timing
 #          between four groups of 4 / 1 / 2 waves.
 CLASS_TILES_16 = {1: (7, 8, 9, 12, 13, 14, 15, 18, 19, 20, 28, 29, 30, 31, 32, 33, 34, 35), 2: (16, 17, 22, 23, 24, 25),
                   4: (21, 26, 27)}
-CANDIDATES_32 = (2, 3, 4)  # fp32: class 1 only
+CANDIDATES_32 = (2, 3, 4, 6)  # fp32 class 1: 128x128, 256x128, 64x64, 128x64
+SPLIT_32 = (5,)               # fp32 class 4: 32x32, four one-wave K groups
 MAX_ENTRIES = 256
 M_BUCKET = 64
 
@@ -76,7 +80,8 @@ _choice: "OrderedDict[Tuple, int]" = OrderedDict()
 def k_class(m: int, n: int, k: int, dtype: torch.dtype) -> int:
     """K-summation class of the tile used for out[m, n] = a[m, k] w[n, k]^T."""
     if dtype == torch.float32:
-        return 1
+        tiles64 = ((m + 63) // 64) * ((n + 63) // 64)
+        return 4 if (tiles64 <= 128 and k >= 256) or (tiles64 <= 192 and k >= 2048) else 1
     if ((m + 31) // 32) * ((n + 63) // 64) <= 256 and k >= 2048:
         return 4
     one_round = ((m + 127) // 128) * ((n + 63) // 64) <= 256
@@ -85,7 +90,7 @@ def k_class(m: int, n: int, k: int, dtype: torch.dtype) -> int:
 
 def candidates(m: int, n: int, k: int, dtype: torch.dtype) -> Tuple[int, ...]:
     if dtype == torch.float32:
-        return CANDIDATES_32
+        return CANDIDATES_32 if k_class(m, n, k, dtype) == 1 else SPLIT_32
     return CLASS_TILES_16[k_class(m, n, k, dtype)]
 
 
