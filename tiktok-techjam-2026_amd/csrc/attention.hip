@@ -68,13 +68,14 @@ template <> struct PairPack<float> {
   }
 };
 
-template <typename T, int HDP, int NQ, int KS, bool KEYMASK>
-__global__ __launch_bounds__(256 * KS) void flash_fwd_kernel(
+// NQW waves per key split own a query group of NQW * NQ * 32 queries.
+template <typename T, int HDP, int NQ, int KS, bool KEYMASK, int NQW = 4>
+__global__ __launch_bounds__(64 * NQW * KS) void flash_fwd_kernel(
     const T* __restrict__ qkv, int64_t sb, int64_t ss, int64_t sc, int64_t sh,
     T* __restrict__ out, int64_t ld_out, int B, int S, int H, int hd, float scale_log2,
     int causal, const int32_t* __restrict__ lengths, const uint8_t* __restrict__ key_mask,
     const int32_t* __restrict__ cu_seqlens, int nqb) {
-  constexpr int NQW = 4;                // waves per key split (one query group each)
+  constexpr int NTS = 64 * NQW;         // threads per key split
   constexpr int BMQ = NQW * NQ * 32;    // queries per workgroup
   constexpr int BNK = 64;               // keys per tile
   constexpr int VEC = 16 / sizeof(T);   // elements per 16-byte chunk
@@ -85,7 +86,7 @@ __global__ __launch_bounds__(256 * KS) void flash_fwd_kernel(
   constexpr int CH = HDP / VEC;         // 16-byte chunks per K/V row
   constexpr int KITEMS = BNK * CH;      // K chunks per tile
   constexpr int VITEMS = (BNK / 2) * CH;  // (key pair, chunk) items per tile
-  static_assert(KITEMS % 256 == 0, "K tile must split evenly over 256 threads");
+  static_assert(KITEMS % NTS == 0, "K tile must split evenly over a split's threads");
 
   __shared__ __attribute__((aligned(16))) T sK[2][KS][BNK * LDK];
   __shared__ __attribute__((aligned(16))) T sV[2][KS][HDP * LDV];
@@ -99,7 +100,7 @@ __global__ __launch_bounds__(256 * KS) void flash_fwd_kernel(
   // Key split: waves qw and qw + NQW*p share query group qw; split p takes
   // key tiles p, p + KS, p + 2 KS, ...; the ltid-th thread of each split
   // stages that split's tiles.
-  const int qw = wave % NQW, par = wave / NQW, ltid = tid & 255;
+  const int qw = wave % NQW, par = wave / NQW, ltid = tid % NTS;
 
   // Sequence b: its tokens are rows row0 .. row0 + Sb - 1 (packed varlen
   // layout when cu_seqlens is given, else b*S .. b*S + S - 1).
@@ -142,21 +143,21 @@ __global__ __launch_bounds__(256 * KS) void flash_fwd_kernel(
   }
 
   // ---- staging of one K/V tile through registers
-  constexpr int KPT = KITEMS / 256;
-  constexpr int VPT = (VITEMS + 255) / 256;
+  constexpr int KPT = KITEMS / NTS;
+  constexpr int VPT = (VITEMS + NTS - 1) / NTS;
   uint4 rk[KPT], rv0[VPT], rv1[VPT];
   auto load_kv = [&](int it) {
     const int k0 = (it * KS + par) * BNK;
 #pragma unroll
     for (int i = 0; i < KPT; ++i) {
-      const int it = ltid + i * 256, key = it / CH, c = it % CH;
+      const int it = ltid + i * NTS, key = it / CH, c = it % CH;
       const int gk = k0 + key, col = c * VEC;
       rk[i] = (gk < Sb && col < hd) ? *reinterpret_cast<const uint4*>(kbase + (int64_t)gk * ss + col)
                                   : make_uint4(0, 0, 0, 0);
     }
 #pragma unroll
     for (int i = 0; i < VPT; ++i) {
-      const int it = ltid + i * 256;
+      const int it = ltid + i * NTS;
       const int p = it % (BNK / 2), c = it / (BNK / 2);
       const int gk = k0 + 2 * p, col = c * VEC;
       const bool ok = it < VITEMS && col < hd;
@@ -169,12 +170,12 @@ __global__ __launch_bounds__(256 * KS) void flash_fwd_kernel(
   auto store_kv = [&](int buf) {
 #pragma unroll
     for (int i = 0; i < KPT; ++i) {
-      const int it = ltid + i * 256, key = it / CH, c = it % CH;
+      const int it = ltid + i * NTS, key = it / CH, c = it % CH;
       *reinterpret_cast<uint4*>(&sK[buf][par][key * LDK + c * VEC]) = rk[i];
     }
 #pragma unroll
     for (int i = 0; i < VPT; ++i) {
-      const int it = ltid + i * 256;
+      const int it = ltid + i * NTS;
       if (it < VITEMS) {
         const int p = it % (BNK / 2), c = it / (BNK / 2);
         PairPack<T>::write(&sV[buf][par][(c * VEC) * LDV + 2 * p], LDV, rv0[i], rv1[i]);
@@ -1525,22 +1526,22 @@ static int launch_pipe(const void* qkv, int64_t sb, int64_t ss, int64_t sc, int6
   return check_launch("tjk_flash_fwd");
 }
 
-template <typename T, int HDP, int NQ, int KS>
+template <typename T, int HDP, int NQ, int KS, int NQW = 4>
 static int launch_flash(const void* qkv, int64_t sb, int64_t ss, int64_t sc, int64_t sh, void* out,
                         int64_t ld_out, int B, int S, int H, int hd, float scale_log2, int causal,
                         const int32_t* lengths, const uint8_t* key_mask, const int32_t* cu_seqlens,
                        hipStream_t st) {
-  constexpr int BMQ = 4 * NQ * 32;
+  constexpr int BMQ = NQW * NQ * 32;
   const int nqb = (S + BMQ - 1) / BMQ;
-  const dim3 block(256 * KS);
+  const dim3 block(64 * NQW * KS);
   const int64_t nblk = (int64_t)nqb * B * H;
   if (nblk > INT32_MAX) return fail(TJK_EUNSUPPORTED, "tjk_flash_fwd: grid too large");
   if (key_mask != nullptr)
-    hipLaunchKernelGGL((flash_fwd_kernel<T, HDP, NQ, KS, true>), dim3((unsigned)nblk), block, 0, st,
+    hipLaunchKernelGGL((flash_fwd_kernel<T, HDP, NQ, KS, true, NQW>), dim3((unsigned)nblk), block, 0, st,
                        (const T*)qkv, sb, ss, sc, sh, (T*)out, ld_out, B, S, H, hd, scale_log2, causal,
                        lengths, key_mask, cu_seqlens, nqb);
   else
-    hipLaunchKernelGGL((flash_fwd_kernel<T, HDP, NQ, KS, false>), dim3((unsigned)nblk), block, 0, st,
+    hipLaunchKernelGGL((flash_fwd_kernel<T, HDP, NQ, KS, false, NQW>), dim3((unsigned)nblk), block, 0, st,
                        (const T*)qkv, sb, ss, sc, sh, (T*)out, ld_out, B, S, H, hd, scale_log2, causal,
                        lengths, key_mask, cu_seqlens, nqb);
   return check_launch("tjk_flash_fwd");
@@ -1565,6 +1566,10 @@ static int launch_short(const void* qkv, int64_t sb, int64_t ss, int64_t sc, int
   return check_launch("tjk_flash_fwd");
 }
 
+// Internal plan (fp32, head_dim <= 64): plan 3 with two waves of queries
+// instead of four, 64 queries and 4 waves per workgroup.
+constexpr int kFaNarrow = 5;
+
 template <typename T, int HDP>
 static int flash_plan(int plan, const void* qkv, int64_t sb, int64_t ss, int64_t sc, int64_t sh, void* out,
                       int64_t ld_out, int B, int S, int H, int hd, float scale_log2, int causal,
@@ -1581,6 +1586,11 @@ static int flash_plan(int plan, const void* qkv, int64_t sb, int64_t ss, int64_t
     if (plan == 4)
       return launch_short<T, HDP>(qkv, sb, ss, sc, sh, out, ld_out, B, S, H, hd, scale_log2, causal, lengths,
                                   key_mask, cu_seqlens, st);
+  }
+  if constexpr (sizeof(T) == 4 && HDP <= 64) {
+    if (plan == kFaNarrow)
+      return launch_flash<T, HDP, 1, 2, 2>(qkv, sb, ss, sc, sh, out, ld_out, B, S, H, hd, scale_log2, causal, lengths,
+                                           key_mask, cu_seqlens, st);
   }
   if (plan == 2)
     return launch_flash<T, HDP, 2, 1>(qkv, sb, ss, sc, sh, out, ld_out, B, S, H, hd, scale_log2, causal, lengths,
@@ -1662,13 +1672,25 @@ extern "C" int tjk_flash_fwd(const void* qkv, int64_t stride_b, int64_t stride_s
   // one-wave workgroup per 32 queries) takes every sequence of at most 128
   // tokens.
   const bool pipe_ok = dtype != TJK_F32 && ((int64_t)seq * stride_s + head_dim) * dtype_size(dtype) < INT32_MAX;
-  if (plan_id == -1) {
+  const bool by_rule = plan_id == -1;
+  if (by_rule) {
     if (seq <= 128)
       plan_id = 4;
     else
       plan_id = (pipe_ok && (key_mask == nullptr || flash_lists(head_dim, seq) || seq < 2048)) ? 0 : 1;
   }
   if (plan_id == 0 && !pipe_ok) plan_id = 1;
+  // fp32 at head_dim <= 64 (matrix-bound: one wave's query block is a serial
+  // chain of 64-cycle MFMAs): 64-query workgroups with two key splits while
+  // 128-query ones would leave CUs idle, else two key splits of 128 queries
+  // for causal sequences past 256 keys.  Measured (us; this / plan 1 / plan 3):
+  // 4 x 512 x 8 heads causal 27.6 / 43.0 / 41.3, 1 x 4096 x 8 199 / 307 / 289;
+  // 2 x 2048 x 16 (512 workgroups of 128) 209 / 212 / 166, 8 x 512 x 12 58 / 59
+  // / 49, not causal 81 / 77 / 84, 16 x 160 x 12 causal 27.8 / 27.9 / 32.3.
+  if (plan_id == 1 && by_rule && dtype == TJK_F32 && head_dim <= 64) {
+    if ((int64_t)((seq + 127) / 128) * batch * heads <= 256) plan_id = kFaNarrow;
+    else if (causal && seq > 256) plan_id = 3;
+  }
   const float scale_log2 = scale * 1.4426950408889634f;
   hipStream_t st = reinterpret_cast<hipStream_t>(stream);
   switch (dtype) {
