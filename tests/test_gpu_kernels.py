@@ -569,6 +569,35 @@ def _attn_ref(qkv, causal, key_mask=None):
 
 
 @pytest.mark.parametrize("causal", [True, False])
+@pytest.mark.parametrize("dt", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("hd", [8, 24, 32, 56, 72, 80, 96, 104, 120])
+def test_flash_head_dims(device, dt, hd, causal):
+    """Plan 0 at head dims below the width its rows have in LDS (32, 64, 96 or
+    128 columns computed), packed lengths around the 64-key tiles and 128- /
+    256-query blocks, whole and through a work list; every row against fp64.
+    The buffer's columns past the last head are NaN."""
+    from tjkernels import schedule
+    heads, lens = 3, [1, 63, 64, 129, 257, 400]
+    g = _gen(hd)
+    t = sum(lens)
+    wide = torch.full((t, 3 * heads * hd + 16), float("nan"), dtype=dt)
+    wide[:, :3 * heads * hd] = torch.randn(t, 3 * heads * hd, generator=g).to(dt)
+    qkv = wide.to(device)[:, :3 * heads * hd].unflatten(1, (3, heads, hd))
+    cu = torch.tensor([0] + torch.tensor(lens).cumsum(0).tolist(), dtype=torch.int32, device=device)
+    rows = qkv.cpu()
+    ref = torch.cat([_attn_ref(rows[a:b].unsqueeze(0), causal) for a, b in zip(cu.tolist(), cu.tolist()[1:])])
+    sched = schedule.build_schedule(lens, heads, hd, causal, dt, device, slots=16)
+    for name in ("grid", "sched"):
+        out = torch.full((t, heads * hd), float("nan"), dtype=dt, device=device)
+        if name == "grid":
+            ops.flash_attention(qkv, out, causal=causal, plan=0, cu_seqlens=cu, max_seqlen=max(lens))
+        else:
+            ops.flash_attention_sched(qkv, out, cu, max(lens), sched, causal=causal)
+        torch.cuda.synchronize()
+        _close(out, ref, OUT_RTOL[dt], 4e-3 if dt == torch.bfloat16 else 1e-3)
+
+
+@pytest.mark.parametrize("causal", [True, False])
 @pytest.mark.parametrize("hd", [24, 64])
 @pytest.mark.parametrize("batch,seq,heads", [(2, 129, 2), (1, 192, 3), (2, 515, 2), (22, 260, 4)])
 def test_flash_fp32_default_plan(device, batch, seq, heads, hd, causal):
@@ -597,12 +626,11 @@ def test_flash_fp32_default_plan(device, batch, seq, heads, hd, causal):
 
 
 @pytest.mark.parametrize("causal", [True, False])
-@pytest.mark.parametrize("hd", [64, 128])
+@pytest.mark.parametrize("hd", [24, 64, 80, 128])
 @pytest.mark.parametrize("dt,seq,heads", [(torch.bfloat16, 129, 2), (torch.float16, 256, 1), (torch.bfloat16, 515, 2),
                                           (torch.float16, 8064, 1), (torch.bfloat16, 8065, 1)])
 def test_flash_masked_lists_keys(device, dt, seq, heads, hd, causal):
-    """Masked plan 0 over the admissible keys only (head_dim 64 / 128, up to
-    8064 keys; one more runs the kernel that masks tiles): every key, none,
+    """Masked plan 0 over the admissible keys only (up to 8064 keys; one more runs the kernel that masks tiles): every key, none,
     a quarter missing, one at either end, whole 64-key blocks missing, exactly
     64 and 65 keys; and with prefix lengths on top.  K of the masked keys is
     NaN: only the admissible keys may enter."""

@@ -566,7 +566,17 @@ __device__ __forceinline__ void fa_lds_dma16(u32x4 rsrc, uint32_t voff, uint32_t
 // into LDS serves 256 queries instead of 128.  Its K and V fragments are
 // read just before use (in two halves for S) to stay within the 256
 // registers two waves per SIMD leave each wave.
-template <typename T, int HDP, bool KEYMASK, bool FULLHD, int NW>
+//
+// HDP is the width of a K / V row in LDS, HDC the head-dim columns computed
+// (32, 64, 96 or 128 for head_dim up to that; HDP 64, 64, 128, 128).  Columns
+// of a row from head_dim on are copied from outside the buffer range: zeros.
+// Measured against the register-staged ring that served head_dim 32 (32-column
+// rows) and 96 (128 columns computed) before: 4 x 2048 x 16 heads, bf16
+// causal, 40.0 -> 37.4 us at 32, 77.8 -> 65.9 at 96; with a key mask 72 -> 41
+// and 212 -> 62.
+enum { kMaskNone = 0, kMaskList = 1, kMaskBytes = 2 };
+
+template <typename T, int HDP, int HDC, int MASK, int NW>
 __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(HDP <= 64 || NW == 8 ? 2 : 1, HDP <= 64 || NW == 8 ? 2 : 1))) void flash_pipe_kernel(
     const T* __restrict__ qkv, int64_t sb, int64_t ss, int64_t sc, int64_t sh,
     T* __restrict__ out, int64_t ld_out, int B, int S, int H, int hd, float scale_log2,
@@ -579,19 +589,20 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(HDP <= 
   constexpr int NT = 64 * NW, BMQ = 32 * NW, BNK = 64, NST = 4, VEC = 8;
   constexpr bool LEAN = NW == 8;  // fragments read just before use
   constexpr int LDK = HDP + VEC, LDV = BNK + VEC;
-  constexpr int KC = HDP / 16, HB = HDP / 32, CH = HDP / VEC;
+  constexpr int KC = HDC / 16, HB = HDC / 32, CH = HDP / VEC;
+  constexpr int PW = HDC == 96 ? 128 : HDC;  // row width of a published partial
   constexpr int KITEMS = BNK * CH, VITEMS = (BNK / 2) * CH;
   constexpr int KPT = KITEMS / NT, VPT = (VITEMS + NT - 1) / NT;
   static_assert(KITEMS % NT == 0, "K tile must split evenly over the threads");
 
-  // K / V ring.  DMA (head_dim 64 / 128 with the full head dimension): tiles
-  // are copied straight into LDS by buffer_load ... lds, K
-  // and V both key-major with 128- / 256-byte rows whose 16-byte chunks are
-  // XOR-swizzled by row, and V^T fragments are gathered with the transposing
-  // ds_read_b64_tr_b16.  Otherwise tiles pass through registers, V stored
-  // transposed.
-  constexpr bool DMA = FULLHD && HDP >= 64;
-  // LIST (DMA ring with a key mask): the workgroup lists its admissible keys
+  // K / V ring.  DMA: tiles are copied straight into LDS by buffer_load ...
+  // lds, K and V both key-major with 128- / 256-byte rows whose 16-byte chunks
+  // are XOR-swizzled by row, and V^T fragments are gathered with the
+  // transposing ds_read_b64_tr_b16.  Otherwise (a key mask too long to list)
+  // tiles pass through registers, V stored transposed.
+  constexpr bool DMA = MASK != kMaskBytes, KEYMASK = MASK == kMaskBytes;
+  static_assert(!DMA || HDP >= 64, "rows of whole 8-chunk XOR groups");
+  // LIST (a key mask): the workgroup lists its admissible keys
   // first and the ring's tiles hold those keys only, 64 of them each, so the
   // tiles need no mask bytes, run the interior loop up to the diagonal, and
   // masked keys cost nothing.  Key limits (kend, lim, ...) then count listed
@@ -600,7 +611,7 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(HDP <= 
   // 8 x 512 x 12 heads of 64, fp16, 27.6 -> 16.4 us (14.0 without a mask); 4 x
   // 2048 x 16 heads of 64, bf16 causal, 109 (plan 1) -> 48 us (47); 2 x 4096 x
   // 16 heads of 128, causal, 406 -> 114 us (137).
-  constexpr bool LIST = DMA && KEYMASK;
+  constexpr bool LIST = MASK == kMaskList;
   constexpr int RB = HDP * (int)sizeof(T);  // DMA: bytes per K / V row
   constexpr int CPR = RB / 16, RPI = 64 / CPR, TILE_B = BNK * RB;
   char* smem;  // DMA ring: slot st holds K at st * 2 TILE_B, V TILE_B later
@@ -723,7 +734,7 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(HDP <= 
 #pragma unroll
     for (int c = 0; c < KC; ++c) {
       const int col = 16 * c + 8 * hi;
-      if (q < Sb && (FULLHD || col < hd)) {
+      if (q < Sb && col < hd) {
         qf[c] = Mfma<T>::load(qbase + (int64_t)q * ss + col);
       } else {
         float z[8] = {0, 0, 0, 0, 0, 0, 0, 0};
@@ -751,7 +762,7 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(HDP <= 
       const int it = tid + i * NT, key = it / CH, c = it % CH;
       const uint32_t off = (uint32_t)key * row_bytes + (uint32_t)(c * 16);
       uint4 v = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(rsk, off, 0, 0));
-      rk[i] = (FULLHD || c * VEC < hd) ? v : make_uint4(0, 0, 0, 0);
+      rk[i] = c * VEC < hd ? v : make_uint4(0, 0, 0, 0);
     }
 #pragma unroll
     for (int i = 0; i < VPT; ++i) {
@@ -760,7 +771,7 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(HDP <= 
       const uint32_t off = (uint32_t)(2 * p) * row_bytes + (uint32_t)(c * 16);
       uint4 v0 = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(rsv, off, 0, 0));
       uint4 v1 = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(rsv, off + row_bytes, 0, 0));
-      const bool ok = FULLHD || c * VEC < hd;
+      const bool ok = c * VEC < hd;
       rv0[i] = ok ? v0 : make_uint4(0, 0, 0, 0);
       rv1[i] = ok ? v1 : make_uint4(0, 0, 0, 0);
     }
@@ -811,12 +822,14 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(HDP <= 
     const int r0 = r & 1, r1 = (r >> 1) & 1, r2 = (r >> 2) & 1, r3 = (r >> 3) & 1;
     return CPR == 8 ? (r1 | (r3 << 1) | ((r1 ^ r2) << 2)) : (r0 | (r1 << 1) | ((r0 ^ r2) << 2) | ((r1 ^ r3) << 3));
   };
+  constexpr uint32_t kPastRange = 0x80000000u;  // beyond any descriptor's range: zeros
   uint32_t dvoff[NDK];
   const uint32_t lds_ring = (uint32_t)(uintptr_t)(lds_void*)smem;
 #pragma unroll
   for (int q = 0; q < NDK; ++q) {
     const int r = (q * NW + wave) * RPI + lane / CPR;
-    dvoff[q] = (uint32_t)r * row_bytes + (uint32_t)(((lane % CPR) ^ swz(r)) << 4);
+    const int c = (lane % CPR) ^ swz(r);
+    dvoff[q] = (LIST ? 0 : (uint32_t)r * row_bytes) + (c * VEC < hd ? (uint32_t)(c << 4) : kPastRange);
   }
   // LIST: this lane's listed key of each DMA instruction of the tile that is
   // copied next, read from the list one tile ahead
@@ -836,8 +849,7 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(HDP <= 
 #pragma unroll
       for (int q = 0; q < NDK; ++q) {
         const int r = (q * NW + wave) * RPI + lane / CPR;
-        off[q] = t * BNK + r < kend ? (uint32_t)dkey[q] * row_bytes + (uint32_t)(((lane % CPR) ^ swz(r)) << 4)
-                                    : 0x80000000u;  // past the list, and any range: zeros
+        off[q] = t * BNK + r < kend ? (uint32_t)dkey[q] * row_bytes + dvoff[q] : kPastRange;
       }
 #pragma unroll
       for (int q = 0; q < NDK; ++q) fa_lds_dma16(rk, off[q], kb + q * NW * 1024);
@@ -884,15 +896,15 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(HDP <= 
   // ch = 4 hb + 2 b4 + b1 (b1 = (lane & 3) >> 1), 8-byte half lane & 1.  In
   // ch ^ swz(key) the bits below 2 depend on the lane only, and the bits from
   // 2 up are c ^ x, c = hb ^ rd for every lane and x a per-lane value, so the
-  // address is one of HB per-lane bases (by c) plus a compile-time offset.
+  // address is one of HDP / 32 per-lane bases (by c) plus a compile-time offset.
   const int vg = (lane & 15) >> 2, g0 = vg & 1, g1 = vg >> 1;
   const int b4 = (lane >> 4) & 1, b1 = (lane & 3) >> 1;
   const int vlow = CPR == 8 ? ((b1 ^ g1) | ((b4 ^ hi) << 1)) : ((b1 ^ g0) | ((b4 ^ g1) << 1));
   const int vx = CPR == 8 ? g1 : (g0 | ((g1 ^ hi) << 1));
   const int vlb = (8 * hi + vg) * RB + 16 * vlow + 8 * (lane & 1);
-  int vlane[HB];
+  int vlane[HDP / 32];
 #pragma unroll
-  for (int c = 0; c < HB; ++c) vlane[c] = vlb + 64 * (c ^ vx);
+  for (int c = 0; c < HDP / 32; ++c) vlane[c] = vlb + 64 * (c ^ vx);
   auto vfrag = [&](int st, int hb, int stp) __attribute__((always_inline)) -> FragT {
     if constexpr (DMA) {
       typedef short v4s __attribute__((ext_vector_type(4)));
@@ -1190,7 +1202,7 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(HDP <= 
   if (t_hi > t_lo) qk(0, scur);
   // Interior tiles: every key below the workgroup's first query and inside
   // the sequence, and a next tile exists in this item's range.
-  int n_int = KEYMASK && !LIST ? 0 : min(causal ? lim_wg / BNK : nkt, min(kend / BNK, t_hi - 1));
+  int n_int = KEYMASK ? 0 : min(causal ? lim_wg / BNK : nkt, min(kend / BNK, t_hi - 1));
   n_int = max(n_int, t_lo);
   int t = t_lo;
   // an unmasked first tile starts the offset at its row max, so the
@@ -1250,7 +1262,7 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(HDP <= 
     if (act) {
       // a tile below the wave's first query and inside the sequence (the
       // first diagonal tile for the upper waves) needs no mask
-      if ((KEYMASK && !LIST) || (causal && t * BNK + BNK > lim_lo) || t * BNK + BNK > kend) mask_tile(t, scur);
+      if (KEYMASK || (causal && t * BNK + BNK > lim_lo) || t * BNK + BNK > kend) mask_tile(t, scur);
       softmax_pv(slot_of(t), scur);
     }
     step_barrier();
@@ -1266,15 +1278,15 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(HDP <= 
   const int q = wq0 + l32;
   const auto lsw = __builtin_amdgcn_permlane32_swap(__float_as_uint(l_run), __float_as_uint(l_run), false, false);
   const float l = __uint_as_float(lsw[0]) + __uint_as_float(lsw[1]);
-  // Partial slot s: O^T rows [query][HDP] fp32, then m[BMQ], then l[BMQ].
+  // Partial slot s: O^T rows [query][PW] fp32, then m[BMQ], then l[BMQ].
   // The halves of a split item are different workgroups, possibly on
   // different XCDs: the partial is written through to memory (sc0 sc1) and
   // read device-coherently (sc1), with a flag per slot in between.
   // The descriptor covers exactly the n_slots partial slots.
   const __amdgpu_buffer_rsrc_t prs =
-      __builtin_amdgcn_make_buffer_rsrc(partials, (short)0, n_slots * (BMQ * (HDP + 2)) * 4, 0x00020000);
-  auto pslot = [&](int sl) { return sl * (BMQ * (HDP + 2)) * 4; };  // byte offset
-  const int prow = (wave * 32 + l32) * HDP * 4;
+      __builtin_amdgcn_make_buffer_rsrc(partials, (short)0, n_slots * (BMQ * (PW + 2)) * 4, 0x00020000);
+  auto pslot = [&](int sl) { return sl * (BMQ * (PW + 2)) * 4; };  // byte offset
+  const int prow = (wave * 32 + l32) * PW * 4;
   if (slot >= 0) {
     const int pb = pslot(slot);
 #pragma unroll
@@ -1287,9 +1299,9 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(HDP <= 
       }
     if (hi == 0) {
       __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, m_off), prs,
-                                            pb + (BMQ * HDP + wave * 32 + l32) * 4, 0, kFaSc0Sc1);
+                                            pb + (BMQ * PW + wave * 32 + l32) * 4, 0, kFaSc0Sc1);
       __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, l), prs,
-                                            pb + (BMQ * HDP + BMQ + wave * 32 + l32) * 4, 0, kFaSc0Sc1);
+                                            pb + (BMQ * PW + BMQ + wave * 32 + l32) * 4, 0, kFaSc0Sc1);
     }
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the partial is in memory
     __syncthreads();
@@ -1338,9 +1350,9 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(HDP <= 
   if (slot <= -2 && merged) {
     const int ps = -2 - slot, pb = pslot(ps);
     const float m_lo = __builtin_bit_cast(
-        float, __builtin_amdgcn_raw_buffer_load_b32(prs, pb + (BMQ * HDP + wave * 32 + l32) * 4, 0, kFaSc1));
+        float, __builtin_amdgcn_raw_buffer_load_b32(prs, pb + (BMQ * PW + wave * 32 + l32) * 4, 0, kFaSc1));
     const float l_lo = __builtin_bit_cast(
-        float, __builtin_amdgcn_raw_buffer_load_b32(prs, pb + (BMQ * HDP + BMQ + wave * 32 + l32) * 4, 0, kFaSc1));
+        float, __builtin_amdgcn_raw_buffer_load_b32(prs, pb + (BMQ * PW + BMQ + wave * 32 + l32) * 4, 0, kFaSc1));
     const float m = fmaxf(m_lo, m_off);
     const float a_lo = m_lo == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(m_lo - m);
     const float a_hi = m_off == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(m_off - m);
@@ -1361,12 +1373,12 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(HDP <= 
       __hip_atomic_fetch_add(&flags[-1], 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     inv = __builtin_nanf("");
   }
-  // DMA ring: the wave's 32 x HDP block goes through LDS and out as 16-byte
+  // DMA ring: the wave's 32 x HDC block goes through LDS and out as 16-byte
   // pieces of whole rows, 8 lanes per 128 bytes, so a launch that writes 4
   // MiB or more can write them through the L2 (its 8-byte pieces 2 KB apart,
   // stored straight from the accumulator layout, measured 4 us slower per C4
   // launch written through, one by one).  Needs 16-byte aligned rows.
-  const bool staged = DMA && ((uintptr_t)out & 15) == 0 && (ld_out % 8) == 0;
+  const bool staged = DMA && hd == HDC && ((uintptr_t)out & 15) == 0 && (ld_out % 8) == 0;
   if (staged) {
     // The ring is free once every wave's copies have landed (the copies of
     // tiles past the item write zeros too) and every wave is past its last
@@ -1374,12 +1386,14 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(HDP <= 
     __syncthreads();
     // The GEMM epilogue's staging layout: whole 16-byte pieces per lane (the
     // halves of pieces g = 2k, 2k + 1 trade lanes l32 and l32 + 32), piece p
-    // of row r at slot r PPR + (p ^ (r & 7)): no LDS bank conflicts for the
+    // of row r at slot r PPR + (p ^ (r & 7)), with rows of whole groups of 4
+    // pieces only p ^ (r / 2 & 3): no LDS bank conflicts for the
     // 8-lanes-per-cycle writes or the 32-lanes-per-cycle reads.
-    constexpr int PPR = HDP * 2 / 16;            // 16-byte pieces per row (8 or 16)
+    constexpr int PPR = HDC * 2 / 16;            // 16-byte pieces per row (4, 8, 12 or 16)
     constexpr int NPASS = 32 * PPR / 64;         // store instructions per wave
-    static_assert(!DMA || PPR % 8 == 0, "rows of whole 8-piece XOR groups");
-    auto slot = [](int r, int p) __attribute__((always_inline)) { return (r * PPR + (p ^ (r & 7))) * 16; };
+    auto slot = [](int r, int p) __attribute__((always_inline)) {
+      return (r * PPR + (p ^ (PPR % 8 == 0 ? r & 7 : r >> 1 & 3))) * 16;
+    };
     char* stg = smem + wave * 32 * PPR * 16;
     auto scaled = [&](int hb, int g) __attribute__((always_inline)) {
       return Quad<T>::from(make_float4(o[hb][4 * g] * inv, o[hb][4 * g + 1] * inv, o[hb][4 * g + 2] * inv,
@@ -1396,8 +1410,8 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(HDP <= 
       }
     const int nrow = min(Sb - wq0, 32);
     const RowOut rows(out + (row0 + wq0) * ld_out + (int64_t)h * hd,
-                      nrow > 0 ? ((int64_t)(nrow - 1) * ld_out + HDP) * (int64_t)sizeof(T) : 0,
-                      (int64_t)B * S * H * HDP * (int64_t)sizeof(T) >= kWtMinBytes);
+                      nrow > 0 ? ((int64_t)(nrow - 1) * ld_out + HDC) * (int64_t)sizeof(T) : 0,
+                      (int64_t)B * S * H * HDC * (int64_t)sizeof(T) >= kWtMinBytes);
     with_wt(rows.wt, [&](auto wt_tag) {
       const auto w = rows.writer<decltype(wt_tag)::value>();
 #pragma unroll
@@ -1414,7 +1428,7 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(HDP <= 
 #pragma unroll
       for (int g = 0; g < 4; ++g) {
         const int col = hb * 32 + 8 * g + 4 * hi;
-        if (FULLHD || col < hd) {
+        if (col < hd) {
           const float4 v = make_float4(o[hb][4 * g] * inv, o[hb][4 * g + 1] * inv, o[hb][4 * g + 2] * inv,
                                        o[hb][4 * g + 3] * inv);
           *reinterpret_cast<typename Quad<T>::raw*>(orow + col) = Quad<T>::from(v);
@@ -1435,7 +1449,7 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(HDP <= 
   // cannot be placed: it is counted in the error word and dropped.  A slot
   // outside [0, n_slots) (or its second-half image) has no partial to
   // publish or merge: the item's rows are written as NaN and counted.
-  if (!KEYMASK && NW == 4 && work != nullptr) {
+  if (MASK == kMaskNone && NW == 4 && work != nullptr) {
     for (int j = blockIdx.x; j < n_work; j += gridDim.x) {
       const int4 it = work[j];
       if (it.x == -1) continue;
@@ -1464,31 +1478,28 @@ __global__ __launch_bounds__(256) void clear_words_kernel(int* p, int n) {
   for (int i = threadIdx.x; i < n; i += 256) p[i] = 0;
 }
 
-template <typename T, int HDP>
+template <typename T, int HDP, int HDC>
 static int launch_sched(const void* qkv, int64_t ss, int64_t sc, int64_t sh, void* out, int64_t ld_out,
                         int B, int S, int H, int hd, float scale_log2, int causal, const int32_t* cu_seqlens,
                         const int32_t* work, int n_work, int n_lists, float* partials, int n_slots, bool clear,
                         hipStream_t st) {
   // [n_slots partial slots][error word][n_slots flags]; flags[-1] is the error word
-  int* flags = partials != nullptr ? reinterpret_cast<int*>(partials + (size_t)n_slots * 128 * (HDP + 2)) + 1 : nullptr;
+  int* flags = partials != nullptr ? reinterpret_cast<int*>(partials + (size_t)n_slots * 128 * ((HDC == 96 ? 128 : HDC) + 2)) + 1 : nullptr;
   if (clear && flags != nullptr) {
     // a fill kernel, not hipMemsetAsync: the call may be recorded into a graph
     hipLaunchKernelGGL(clear_words_kernel, dim3(1), dim3(256), 0, st, flags - 1, n_slots + 1);
   }
-#define TJK_PIPE_SCHED(FULL)                                                                                  \
-  hipLaunchKernelGGL((flash_pipe_kernel<T, HDP, false, FULL, 4>), dim3((unsigned)n_lists), dim3(256), 0, st,  \
-                     (const T*)qkv, (int64_t)0, ss, sc, sh, (T*)out, ld_out, B, S, H, hd, scale_log2, causal, \
-                     (const int32_t*)nullptr, (const uint8_t*)nullptr, cu_seqlens, 0,                         \
-                     reinterpret_cast<const int4*>(work), n_work, partials, flags, n_slots, 1)
-  if (hd == HDP) TJK_PIPE_SCHED(true); else TJK_PIPE_SCHED(false);
-#undef TJK_PIPE_SCHED
+  hipLaunchKernelGGL((flash_pipe_kernel<T, HDP, HDC, kMaskNone, 4>), dim3((unsigned)n_lists), dim3(256), 0, st,
+                     (const T*)qkv, (int64_t)0, ss, sc, sh, (T*)out, ld_out, B, S, H, hd, scale_log2, causal,
+                     (const int32_t*)nullptr, (const uint8_t*)nullptr, cu_seqlens, 0,
+                     reinterpret_cast<const int4*>(work), n_work, partials, flags, n_slots, 1);
   return check_launch("tjk_flash_fwd_sched");
 }
 
 // Whether a masked launch of plan 0 lists its admissible keys.
-static bool flash_lists(int hd, int S) { return (hd == 64 || hd == 128) && S <= kFaListKeys; }
+static bool flash_lists(int S) { return S <= kFaListKeys; }
 
-template <typename T, int HDP>
+template <typename T, int HDP, int HDC>
 static int launch_pipe(const void* qkv, int64_t sb, int64_t ss, int64_t sc, int64_t sh, void* out,
                        int64_t ld_out, int B, int S, int H, int hd, float scale_log2, int causal,
                        const int32_t* lengths, const uint8_t* key_mask, const int32_t* cu_seqlens,
@@ -1497,7 +1508,7 @@ static int launch_pipe(const void* qkv, int64_t sb, int64_t ss, int64_t sc, int6
   // flash_pipe_kernel), except for masked launches that do not list their keys
   // (that variant would spill)
   constexpr int NW8 = HDP == 128 ? 8 : 4;
-  const bool list = key_mask != nullptr && flash_lists(hd, S);
+  const bool list = key_mask != nullptr && flash_lists(S);
   const int nw = key_mask == nullptr || list ? NW8 : 4;
   const int nqb = (S + 32 * nw - 1) / (32 * nw);
   const int64_t nblk = (int64_t)nqb * B * H;
@@ -1509,18 +1520,17 @@ static int launch_pipe(const void* qkv, int64_t sb, int64_t ss, int64_t sc, int6
   const int64_t kv_pair = (int64_t)S * hd * 2 * (int64_t)sizeof(T);
   const int64_t fit = (int64_t)128 * 1024 * 1024 / (kv_pair > 0 ? kv_pair : 1);
   const int grp = (int)std::max<int64_t>(std::min<int64_t>(B * H, std::max<int64_t>(fit, 8)), 1);
-#define TJK_PIPE(KM, FULL, NWV)                                                                                \
-  hipLaunchKernelGGL((flash_pipe_kernel<T, HDP, KM, FULL, NWV>), dim3((unsigned)nblk), dim3(64 * NWV), 0, st,   \
+#define TJK_PIPE(HP, HC, KM, NWV)                                                                                \
+  hipLaunchKernelGGL((flash_pipe_kernel<T, HP, HC, KM, NWV>), dim3((unsigned)nblk), dim3(64 * NWV), 0, st,   \
                      (const T*)qkv, sb, ss, sc, sh, (T*)out, ld_out, B, S, H, hd, scale_log2, causal, lengths,  \
                      key_mask, cu_seqlens, nqb, (const int4*)nullptr, 0, (float*)nullptr, (int*)nullptr, 0, grp)
-  if (key_mask != nullptr) {
-    if constexpr (HDP >= 64) {
-      if (list) TJK_PIPE(true, true, NW8); else TJK_PIPE(true, false, 4);
-    } else {
-      TJK_PIPE(true, false, 4);
-    }
+  if (key_mask != nullptr && !list) {
+    // (rows of 32, 64 or 128: this variant's tiles are not swizzled)
+    TJK_PIPE((HDC == 32 ? 32 : HDP), (HDC == 32 ? 32 : HDP), kMaskBytes, 4);
+  } else if (key_mask != nullptr) {
+    TJK_PIPE(HDP, HDC, kMaskList, NW8);
   } else {
-    if (hd == HDP) TJK_PIPE(false, true, NW8); else TJK_PIPE(false, false, NW8);
+    TJK_PIPE(HDP, HDC, kMaskNone, NW8);
   }
 #undef TJK_PIPE
   return check_launch("tjk_flash_fwd");
@@ -1576,8 +1586,13 @@ static int flash_plan(int plan, const void* qkv, int64_t sb, int64_t ss, int64_t
                       const int32_t* lengths, const uint8_t* key_mask, const int32_t* cu_seqlens,
                        hipStream_t st) {
   if constexpr (sizeof(T) == 2) {
+    if constexpr (HDP == 128) {
+      if (plan == 0 && hd <= 96)
+        return launch_pipe<T, 128, 96>(qkv, sb, ss, sc, sh, out, ld_out, B, S, H, hd, scale_log2, causal, lengths,
+                                       key_mask, cu_seqlens, st);
+    }
     if (plan == 0)
-      return launch_pipe<T, HDP>(qkv, sb, ss, sc, sh, out, ld_out, B, S, H, hd, scale_log2, causal, lengths,
+      return launch_pipe<T, (HDP < 64 ? 64 : HDP), HDP>(qkv, sb, ss, sc, sh, out, ld_out, B, S, H, hd, scale_log2, causal, lengths,
                                  key_mask, cu_seqlens, st);
   }
   // plan 4: sequences of at most 128 tokens (checked by the entry point);
@@ -1663,10 +1678,10 @@ extern "C" int tjk_flash_fwd(const void* qkv, int64_t stride_b, int64_t stride_s
   // at hd 128 too since its 8-wave workgroups (causal 16 x 512: 50.5 vs
   // 53.0 us, 4 x 2048: 95.1 vs 122.6 us, 2 x 8192: 615 vs 743 us); plans 2
   // and 3 were slower on every BASELINE shape.
-  // With a key mask plan 0 lists the admissible keys where it can (see
-  // flash_pipe_kernel); otherwise it runs every tile through its masked
-  // (unpipelined) loop: plan 1 from S = 2048 (padded C4 with a per-key
-  // mask: 129 vs 168 us).  A sequence of one 128-query block has only
+  // With a key mask plan 0 lists the admissible keys up to kFaListKeys of
+  // them (see flash_pipe_kernel); past that it runs every tile through its
+  // masked (unpipelined) loop, and plan 1 is faster (4 x 2048, hd 64: 129 vs
+  // 168 us).  A sequence of one 128-query block has only
   // diagonal tiles and nothing to pipeline: plan 1 there too (C2's
   // 1 x 128 x 8 heads fp16: 6.2 vs 6.8 us).  Plan 4 (whole sequence in one
   // one-wave workgroup per 32 queries) takes every sequence of at most 128
@@ -1677,7 +1692,7 @@ extern "C" int tjk_flash_fwd(const void* qkv, int64_t stride_b, int64_t stride_s
     if (seq <= 128)
       plan_id = 4;
     else
-      plan_id = (pipe_ok && (key_mask == nullptr || flash_lists(head_dim, seq) || seq < 2048)) ? 0 : 1;
+      plan_id = (pipe_ok && (key_mask == nullptr || flash_lists(seq))) ? 0 : 1;
   }
   if (plan_id == 0 && !pipe_ok) plan_id = 1;
   // fp32 at head_dim <= 64 (matrix-bound: one wave's query block is a serial
@@ -1740,18 +1755,20 @@ static int flash_sched_entry(const char* who, const void* qkv, int64_t stride_s,
     return fail(TJK_EUNSUPPORTED, "%s: misaligned pointer", who);
   if (!(scale > 0.f)) return fail(TJK_EINVAL, "%s: scale must be positive", who);
   const float scale_log2 = scale * 1.4426950408889634f;
-#define TJK_SCHED(TT, HDP)                                                                                  \
-  return launch_sched<TT, HDP>(qkv, stride_s, stride_c, stride_h, out, ld_out, batch, max_seqlen, heads, \
+#define TJK_SCHED(TT, HDP, HDC)                                                                                  \
+  return launch_sched<TT, HDP, HDC>(qkv, stride_s, stride_c, stride_h, out, ld_out, batch, max_seqlen, heads, \
                                head_dim, scale_log2, causal, cu_seqlens, work, n_work, n_lists, partials, n_slots, \
                                clear, st)
   if (dtype == TJK_F16) {
-    if (head_dim <= 32) TJK_SCHED(f16, 32);
-    if (head_dim <= 64) TJK_SCHED(f16, 64);
-    TJK_SCHED(f16, 128);
+    if (head_dim <= 32) TJK_SCHED(f16, 64, 32);
+    if (head_dim <= 64) TJK_SCHED(f16, 64, 64);
+    if (head_dim <= 96) TJK_SCHED(f16, 128, 96);
+    TJK_SCHED(f16, 128, 128);
   }
-  if (head_dim <= 32) TJK_SCHED(bf16, 32);
-  if (head_dim <= 64) TJK_SCHED(bf16, 64);
-  TJK_SCHED(bf16, 128);
+  if (head_dim <= 32) TJK_SCHED(bf16, 64, 32);
+  if (head_dim <= 64) TJK_SCHED(bf16, 64, 64);
+  if (head_dim <= 96) TJK_SCHED(bf16, 128, 96);
+  TJK_SCHED(bf16, 128, 128);
 #undef TJK_SCHED
 }
 
@@ -1825,10 +1842,12 @@ extern "C" int tjk_flash_sched_occupancy(int head_dim, int dtype) {
   int blocks = 0;
   hipError_t e = hipErrorInvalidValue;
   const bool h16 = dtype == TJK_F16;
-#define TJK_OCC(TT, HDP) e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&blocks, flash_pipe_kernel<TT, HDP, false, true, 4>, 256, 0)
-  if (head_dim <= 32) { if (h16) TJK_OCC(f16, 32); else TJK_OCC(bf16, 32); }
-  else if (head_dim <= 64) { if (h16) TJK_OCC(f16, 64); else TJK_OCC(bf16, 64); }
-  else { if (h16) TJK_OCC(f16, 128); else TJK_OCC(bf16, 128); }
+#define TJK_OCC(TT, HDP, HDC) \
+  e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&blocks, flash_pipe_kernel<TT, HDP, HDC, kMaskNone, 4>, 256, 0)
+  if (head_dim <= 32) { if (h16) TJK_OCC(f16, 64, 32); else TJK_OCC(bf16, 64, 32); }
+  else if (head_dim <= 64) { if (h16) TJK_OCC(f16, 64, 64); else TJK_OCC(bf16, 64, 64); }
+  else if (head_dim <= 96) { if (h16) TJK_OCC(f16, 128, 96); else TJK_OCC(bf16, 128, 96); }
+  else { if (h16) TJK_OCC(f16, 128, 128); else TJK_OCC(bf16, 128, 128); }
 #undef TJK_OCC
   if (e != hipSuccess) return fail(hip_status(e), "tjk_flash_sched_occupancy: %s", hipGetErrorString(e));
   return blocks;
