@@ -574,7 +574,8 @@ __device__ __forceinline__ void fa_lds_dma16(u32x4 rsrc, uint32_t voff, uint32_t
 // rows) and 96 (128 columns computed) before: 4 x 2048 x 16 heads, bf16
 // causal, 40.0 -> 37.4 us at 32, 77.8 -> 65.9 at 96; with a key mask 72 -> 41
 // and 212 -> 62.
-enum { kMaskNone = 0, kMaskList = 1, kMaskBytes = 2 };
+// kMaskBytesFull: kMaskBytes with head_dim == HDC.
+enum { kMaskNone = 0, kMaskList = 1, kMaskBytes = 2, kMaskBytesFull = 3 };
 
 template <typename T, int HDP, int HDC, int MASK, int NW>
 __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(HDP <= 64 || NW == 8 ? 2 : 1, HDP <= 64 || NW == 8 ? 2 : 1))) void flash_pipe_kernel(
@@ -598,9 +599,9 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(HDP <= 
   // K / V ring.  DMA: tiles are copied straight into LDS by buffer_load ...
   // lds, K and V both key-major with 128- / 256-byte rows whose 16-byte chunks
   // are XOR-swizzled by row, and V^T fragments are gathered with the
-  // transposing ds_read_b64_tr_b16.  Otherwise (a key mask too long to list)
+  // transposing ds_read_b64_tr_b16.  Otherwise (a key mask that is not listed)
   // tiles pass through registers, V stored transposed.
-  constexpr bool DMA = MASK != kMaskBytes, KEYMASK = MASK == kMaskBytes;
+  constexpr bool FULLHD = MASK == kMaskBytesFull, KEYMASK = MASK == kMaskBytes || FULLHD, DMA = !KEYMASK;
   static_assert(!DMA || HDP >= 64, "rows of whole 8-chunk XOR groups");
   // LIST (a key mask): the workgroup lists its admissible keys
   // first and the ring's tiles hold those keys only, 64 of them each, so the
@@ -734,7 +735,7 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(HDP <= 
 #pragma unroll
     for (int c = 0; c < KC; ++c) {
       const int col = 16 * c + 8 * hi;
-      if (q < Sb && col < hd) {
+      if (q < Sb && (FULLHD || col < hd)) {
         qf[c] = Mfma<T>::load(qbase + (int64_t)q * ss + col);
       } else {
         float z[8] = {0, 0, 0, 0, 0, 0, 0, 0};
@@ -762,7 +763,7 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(HDP <= 
       const int it = tid + i * NT, key = it / CH, c = it % CH;
       const uint32_t off = (uint32_t)key * row_bytes + (uint32_t)(c * 16);
       uint4 v = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(rsk, off, 0, 0));
-      rk[i] = c * VEC < hd ? v : make_uint4(0, 0, 0, 0);
+      rk[i] = FULLHD || c * VEC < hd ? v : make_uint4(0, 0, 0, 0);
     }
 #pragma unroll
     for (int i = 0; i < VPT; ++i) {
@@ -771,7 +772,7 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(HDP <= 
       const uint32_t off = (uint32_t)(2 * p) * row_bytes + (uint32_t)(c * 16);
       uint4 v0 = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(rsv, off, 0, 0));
       uint4 v1 = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(rsv, off + row_bytes, 0, 0));
-      const bool ok = c * VEC < hd;
+      const bool ok = FULLHD || c * VEC < hd;
       rv0[i] = ok ? v0 : make_uint4(0, 0, 0, 0);
       rv1[i] = ok ? v1 : make_uint4(0, 0, 0, 0);
     }
@@ -1428,7 +1429,7 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(HDP <= 
 #pragma unroll
       for (int g = 0; g < 4; ++g) {
         const int col = hb * 32 + 8 * g + 4 * hi;
-        if (col < hd) {
+        if (FULLHD || col < hd) {
           const float4 v = make_float4(o[hb][4 * g] * inv, o[hb][4 * g + 1] * inv, o[hb][4 * g + 2] * inv,
                                        o[hb][4 * g + 3] * inv);
           *reinterpret_cast<typename Quad<T>::raw*>(orow + col) = Quad<T>::from(v);
@@ -1496,8 +1497,11 @@ static int launch_sched(const void* qkv, int64_t ss, int64_t sc, int64_t sh, voi
   return check_launch("tjk_flash_fwd_sched");
 }
 
-// Whether a masked launch of plan 0 lists its admissible keys.
-static bool flash_lists(int S) { return S <= kFaListKeys; }
+// Whether a masked launch of plan 0 lists its admissible keys.  Below 256 keys
+// listing them before the first copy costs more than the masked tiles (8 x 12
+// heads of 64, causal: 192 keys 9.4 us masking tiles, 10.0 listing; 256 keys
+// 11.4, 10.8).
+static bool flash_lists(int S) { return S >= 256 && S <= kFaListKeys; }
 
 template <typename T, int HDP, int HDC>
 static int launch_pipe(const void* qkv, int64_t sb, int64_t ss, int64_t sc, int64_t sh, void* out,
@@ -1526,7 +1530,8 @@ static int launch_pipe(const void* qkv, int64_t sb, int64_t ss, int64_t sc, int6
                      key_mask, cu_seqlens, nqb, (const int4*)nullptr, 0, (float*)nullptr, (int*)nullptr, 0, grp)
   if (key_mask != nullptr && !list) {
     // (rows of 32, 64 or 128: this variant's tiles are not swizzled)
-    TJK_PIPE((HDC == 32 ? 32 : HDP), (HDC == 32 ? 32 : HDP), kMaskBytes, 4);
+    constexpr int HB = HDC == 32 ? 32 : HDP;
+    if (hd == HB) TJK_PIPE(HB, HB, kMaskBytesFull, 4); else TJK_PIPE(HB, HB, kMaskBytes, 4);
   } else if (key_mask != nullptr) {
     TJK_PIPE(HDP, HDC, kMaskList, NW8);
   } else {
@@ -1678,10 +1683,10 @@ extern "C" int tjk_flash_fwd(const void* qkv, int64_t stride_b, int64_t stride_s
   // at hd 128 too since its 8-wave workgroups (causal 16 x 512: 50.5 vs
   // 53.0 us, 4 x 2048: 95.1 vs 122.6 us, 2 x 8192: 615 vs 743 us); plans 2
   // and 3 were slower on every BASELINE shape.
-  // With a key mask plan 0 lists the admissible keys up to kFaListKeys of
-  // them (see flash_pipe_kernel); past that it runs every tile through its
-  // masked (unpipelined) loop, and plan 1 is faster (4 x 2048, hd 64: 129 vs
-  // 168 us).  A sequence of one 128-query block has only
+  // With a key mask plan 0 lists the admissible keys of 256 up to kFaListKeys
+  // keys (flash_lists); otherwise it runs every tile through its masked
+  // (unpipelined) loop, and past kFaListKeys plan 1 is faster (4 x 2048, hd 64:
+  // 129 vs 168 us).  A sequence of one 128-query block has only
   // diagonal tiles and nothing to pipeline: plan 1 there too (C2's
   // 1 x 128 x 8 heads fp16: 6.2 vs 6.8 us).  Plan 4 (whole sequence in one
   // one-wave workgroup per 32 queries) takes every sequence of at most 128
@@ -1692,7 +1697,7 @@ extern "C" int tjk_flash_fwd(const void* qkv, int64_t stride_b, int64_t stride_s
     if (seq <= 128)
       plan_id = 4;
     else
-      plan_id = (pipe_ok && (key_mask == nullptr || flash_lists(seq))) ? 0 : 1;
+      plan_id = (pipe_ok && (key_mask == nullptr || seq <= kFaListKeys)) ? 0 : 1;
   }
   if (plan_id == 0 && !pipe_ok) plan_id = 1;
   // fp32 at head_dim <= 64 (matrix-bound: one wave's query block is a serial
