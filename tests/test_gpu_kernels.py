@@ -205,6 +205,26 @@ def test_gemm_panel_plans(device, dt, plan):
         assert torch.equal(*outs), (m, n, k, "from")
 
 
+@pytest.mark.parametrize("m,n,k", [(700, 960, 512), (700, 1024, 512), (700, 1024, 704), (700, 1024, 768),
+                                   (512, 2048, 512), (513, 2048, 512), (1024, 2048, 512), (1025, 2048, 512)])
+def test_gemm_default_tile_keeps_its_class(device, m, n, k):
+    """Without a plan, the bits of the tiles that the timing chooses from, on
+    both sides of the lines between the K-summation classes."""
+    from tjkernels import tiles
+    g = _gen(m + n + k)
+    a = torch.randn(m, k, generator=g).bfloat16().to(device)
+    w = (torch.randn(n, k, generator=g) * k ** -0.5).bfloat16().to(device)
+    bias = torch.randn(n, generator=g).bfloat16().to(device)
+    cls = tiles.candidates(m, n, k, torch.bfloat16)
+    outs = []
+    for plan in (-1, cls[0], cls[-1]):
+        outs.append(torch.empty(m, n, device=device))
+        outs[-1].zero_()
+        ops.gemm(a, w, bias, outs[-1], ops.EPI_BIAS_RESIDUAL, plan)
+    torch.cuda.synchronize()
+    assert torch.equal(outs[0], outs[1]) and torch.equal(outs[0], outs[2])
+
+
 @pytest.mark.parametrize("m,n,k", [  # the tile the default rule takes:
     (1, 4, 8), (70, 68, 200),   # 64 x 64
     (5547, 324, 40),            # 96 x 128

@@ -84,8 +84,8 @@ def k_class(m: int, n: int, k: int, dtype: torch.dtype) -> int:
         return 4 if (tiles64 <= 128 and k >= 256) or (tiles64 <= 192 and k >= 2048) else 1
     if ((m + 31) // 32) * ((n + 63) // 64) <= 256 and k >= 2048:
         return 4
-    one_round = ((m + 127) // 128) * ((n + 63) // 64) <= 256
-    return 2 if one_round and k >= 512 else 1
+    tiles = ((m + 127) // 128) * ((n + 63) // 64)
+    return 2 if tiles <= 256 and k >= 512 and (k >= 768 or n < 1024 or tiles <= 128) else 1
 
 
 def candidates(m: int, n: int, k: int, dtype: torch.dtype) -> Tuple[int, ...]:
