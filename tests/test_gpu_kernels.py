@@ -618,6 +618,31 @@ def test_flash_head_dims(device, dt, hd, causal):
 
 
 @pytest.mark.parametrize("causal", [True, False])
+@pytest.mark.parametrize("dt", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("seq", [129, 200, 515])
+def test_flash_head_dim_32_small_launches(device, seq, dt, causal):
+    """Head dim 32 up to 256 workgroups (tiles through registers) and above
+    (copied): the same bits, padded and with lengths, and both near fp64."""
+    heads, nqb = 4, (seq + 127) // 128
+    small = 256 // (nqb * heads)
+    g = _gen(seq)
+    qkv = torch.randn(small + 1, seq, 3, heads, 32, generator=g).to(dt)
+    lens = torch.randint(0, seq + 1, (small + 1,), generator=g).int()
+    d = qkv.to(device)
+    for kw in ({}, dict(lengths=lens.to(device))):
+        outs = []
+        for b in (small, small + 1):
+            out = torch.full((b * seq, heads * 32), float("nan"), dtype=dt, device=device)
+            ops.flash_attention(d[:b], out, causal=causal, **{k: v[:b] for k, v in kw.items()})
+            outs.append(out)
+        torch.cuda.synchronize()
+        assert torch.equal(outs[0], outs[1][:small * seq])
+        mask = torch.arange(seq)[None, :] < lens[:, None] if kw else None
+        ref = _attn_ref(qkv[:2], causal, mask[:2] if kw else None)
+        _close(outs[0][:2 * seq], ref, OUT_RTOL[dt], 4e-3 if dt == torch.bfloat16 else 1e-3)
+
+
+@pytest.mark.parametrize("causal", [True, False])
 @pytest.mark.parametrize("hd", [24, 64])
 @pytest.mark.parametrize("batch,seq,heads", [(2, 129, 2), (1, 192, 3), (2, 515, 2), (22, 260, 4)])
 def test_flash_fp32_default_plan(device, batch, seq, heads, hd, causal):

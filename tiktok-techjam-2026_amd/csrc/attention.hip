@@ -574,8 +574,9 @@ __device__ __forceinline__ void fa_lds_dma16(u32x4 rsrc, uint32_t voff, uint32_t
 // rows) and 96 (128 columns computed) before: 4 x 2048 x 16 heads, bf16
 // causal, 40.0 -> 37.4 us at 32, 77.8 -> 65.9 at 96; with a key mask 72 -> 41
 // and 212 -> 62.
-// kMaskBytesFull: kMaskBytes with head_dim == HDC.
-enum { kMaskNone = 0, kMaskList = 1, kMaskBytes = 2, kMaskBytesFull = 3 };
+// kMaskBytesFull: kMaskBytes with head_dim == HDC.  kMaskNoneRegs: no mask,
+// head_dim == HDC, tiles through registers (see launch_pipe).
+enum { kMaskNone = 0, kMaskList = 1, kMaskBytes = 2, kMaskBytesFull = 3, kMaskNoneRegs = 4 };
 
 template <typename T, int HDP, int HDC, int MASK, int NW>
 __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(HDP <= 64 || NW == 8 ? 2 : 1, HDP <= 64 || NW == 8 ? 2 : 1))) void flash_pipe_kernel(
@@ -599,9 +600,11 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(HDP <= 
   // K / V ring.  DMA: tiles are copied straight into LDS by buffer_load ...
   // lds, K and V both key-major with 128- / 256-byte rows whose 16-byte chunks
   // are XOR-swizzled by row, and V^T fragments are gathered with the
-  // transposing ds_read_b64_tr_b16.  Otherwise (a key mask that is not listed)
-  // tiles pass through registers, V stored transposed.
-  constexpr bool FULLHD = MASK == kMaskBytesFull, KEYMASK = MASK == kMaskBytes || FULLHD, DMA = !KEYMASK;
+  // transposing ds_read_b64_tr_b16.  Otherwise (a key mask that is not listed,
+  // small launches at head_dim 32) tiles pass through registers, V stored
+  // transposed.
+  constexpr bool FULLHD = MASK == kMaskBytesFull || MASK == kMaskNoneRegs;
+  constexpr bool KEYMASK = MASK == kMaskBytes || MASK == kMaskBytesFull, DMA = !KEYMASK && MASK != kMaskNoneRegs;
   static_assert(!DMA || HDP >= 64, "rows of whole 8-chunk XOR groups");
   // LIST (a key mask): the workgroup lists its admissible keys
   // first and the ring's tiles hold those keys only, 64 of them each, so the
@@ -732,15 +735,17 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(HDP <= 
   typename Mfma<T>::frag qf[KC];
   {
     const int q = wq0 + l32;
+    float z[8] = {0, 0, 0, 0, 0, 0, 0, 0};
 #pragma unroll
-    for (int c = 0; c < KC; ++c) {
-      const int col = 16 * c + 8 * hi;
-      if (q < Sb && (FULLHD || col < hd)) {
-        qf[c] = Mfma<T>::load(qbase + (int64_t)q * ss + col);
-      } else {
-        float z[8] = {0, 0, 0, 0, 0, 0, 0, 0};
-        qf[c] = Mfma<T>::pack(z);
-      }
+    for (int c = 0; c < KC; ++c) qf[c] = Mfma<T>::pack(z);
+    if (FULLHD || hd == HDC) {  // all loads under one branch
+      if (q < Sb)
+#pragma unroll
+        for (int c = 0; c < KC; ++c) qf[c] = Mfma<T>::load(qbase + (int64_t)q * ss + 16 * c + 8 * hi);
+    } else {
+#pragma unroll
+      for (int c = 0; c < KC; ++c)
+        if (q < Sb && 16 * c + 8 * hi < hd) qf[c] = Mfma<T>::load(qbase + (int64_t)q * ss + 16 * c + 8 * hi);
     }
   }
 
@@ -1535,6 +1540,18 @@ static int launch_pipe(const void* qkv, int64_t sb, int64_t ss, int64_t sc, int6
   } else if (key_mask != nullptr) {
     TJK_PIPE(HDP, HDC, kMaskList, NW8);
   } else {
+    // head_dim 32 with at most one workgroup per CU: the latency of each tile
+    // counts, and half of a 64-column row's copies are zeros, so 32-column rows
+    // through registers are faster (bf16 causal, registers / copies: 2 x 200 x 4
+    // heads 6.2 / 6.5 us, 4 x 700 x 8 9.4 / 9.8, 2 x 1500 x 4 15.5 / 16.3); above
+    // that the copies are (16 x 160 x 12 1.02 times, 4 x 2048 x 16 40.0 / 37.4).
+    // The same products and sums in the same order either way.
+    if constexpr (HDC == 32) {
+      if (hd == 32 && nblk <= 256) {
+        TJK_PIPE(32, 32, kMaskNoneRegs, 4);
+        return check_launch("tjk_flash_fwd");
+      }
+    }
     TJK_PIPE(HDP, HDC, kMaskNone, NW8);
   }
 #undef TJK_PIPE
@@ -1702,13 +1719,16 @@ extern "C" int tjk_flash_fwd(const void* qkv, int64_t stride_b, int64_t stride_s
   if (plan_id == 0 && !pipe_ok) plan_id = 1;
   // fp32 at head_dim <= 64 (matrix-bound: one wave's query block is a serial
   // chain of 64-cycle MFMAs): 64-query workgroups with two key splits while
-  // 128-query ones would leave CUs idle, else two key splits of 128 queries
-  // for causal sequences past 256 keys.  Measured (us; this / plan 1 / plan 3):
+  // 128-query ones would leave CUs idle (not causal, where every workgroup
+  // takes as long: while the 64-query ones are at most one per CU), else two
+  // key splits of 128 queries for causal sequences past 256 keys.  Measured (us; this / plan 1 / plan 3):
   // 4 x 512 x 8 heads causal 27.6 / 43.0 / 41.3, 1 x 4096 x 8 199 / 307 / 289;
   // 2 x 2048 x 16 (512 workgroups of 128) 209 / 212 / 166, 8 x 512 x 12 58 / 59
-  // / 49, not causal 81 / 77 / 84, 16 x 160 x 12 causal 27.8 / 27.9 / 32.3.
+  // / 49, not causal 81 / 77 / 84, 16 x 160 x 12 causal 27.8 / 27.9 / 32.3; 8 x 260 x 8
+  // (320 workgroups of 64) not causal 39.9 / 29.2, 4 x 700 x 8 73.4 / 57.5.
   if (plan_id == 1 && by_rule && dtype == TJK_F32 && head_dim <= 64) {
-    if ((int64_t)((seq + 127) / 128) * batch * heads <= 256) plan_id = kFaNarrow;
+    const int bq = causal ? 128 : 64;
+    if ((int64_t)((seq + bq - 1) / bq) * batch * heads <= 256) plan_id = kFaNarrow;
     else if (causal && seq > 256) plan_id = 3;
   }
   const float scale_log2 = scale * 1.4426950408889634f;
