@@ -619,6 +619,11 @@ def test_rocprof_summary_labels_deferred_projections():
     ws2 = "_ZN3tjk14gemm_ws_kernelIDF16bLi192ELi128ELi2ELi4ELi4ELi4ELi2EEEvPKT_lS3_lS3_Pvliii"
     assert rs._gemm_epilogue(ws2) == 2 and rs._kind_ok("gemm_out_residual", ws2)
     assert rs._relabel("gemm_out_residual", ws2) == "gemm_out_residual" and rs._tjk(ws2)
+    # the panel ring <T, FM, FN, EPI>
+    panel2 = "_ZN3tjk17gemm_panel_kernelIDF16bLi4ELi4ELi2EEEvPKT_lS3_lS3_Pvliii"
+    assert rs._relabel("gemm_ffn2_residual", panel2) == "gemm_ffn2_residual"
+    assert rs._relabel("gemm_ffn2_residual", panel2.replace("Li2EE", "Li0EE")) == "gemm_ffn2"
+    assert rs._is_gemm(panel2)
     # the first layer's out-proj adding the input rows (EPI 4) is a residual GEMM as well
     ws4 = "_ZN3tjk14gemm_ws_kernelIDF16bLi192ELi128ELi2ELi4ELi4ELi4ELi4EEEvPKT_lS3_lS3_PvliiiNS_6ResSrcE"
     assert rs._gemm_epilogue(ws4) == 4 and rs._relabel("gemm_out_residual", ws4) == "gemm_out_residual"

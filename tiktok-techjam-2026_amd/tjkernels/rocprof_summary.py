@@ -42,13 +42,13 @@ from typing import Dict, List, Optional, Tuple
 
 # add_layernorm_kernel and add_layernorm_parts_kernel (the split-delta sum
 # after the single-launch FFN) both count as LayerNorm launches; a GEMM
-# launch is the direct-to-LDS kernel or the wave-specialized one
+# launch is the direct-to-LDS kernel, the wave-specialized one or the panel ring
 GEMM, FLASH, LN, FFN = "gemm_dtl_kernel", "flash_", "add_layernorm", "ffn_fused_kernel"
-GEMM_WS = "gemm_ws_kernel"
+GEMM_WS, GEMM_PANEL = "gemm_ws_kernel", "gemm_panel_kernel"
 
 
 def _is_gemm(name: str) -> bool:
-    return GEMM in name or GEMM_WS in name
+    return GEMM in name or GEMM_WS in name or GEMM_PANEL in name
 COPY = "__amd_rocclr_copyBuffer"
 
 
@@ -72,8 +72,12 @@ def _labels(layers: int, fused: bool = False) -> List[str]:
 def _gemm_epilogue(name: str) -> Optional[int]:
     """EPI template argument of a gemm_dtl_kernel<T, BM, BN, WM, WN, BKB,
     STAGES, EPI, KSPLIT> or gemm_ws_kernel<T, BM, BN, WM, WN, STAGES, L, EPI>
-    name, the seventh integer in both (2: residual read-modify-write, 4:
-    residual read from the input x, the first layer's out-proj)."""
+    name, the seventh integer in both, or of a gemm_panel_kernel<T, FM, FN,
+    EPI> name, the third (2: residual read-modify-write, 4: residual read from
+    the input x, the first layer's out-proj)."""
+    if GEMM_PANEL in name:
+        ints = re.findall(r"Li(\d+)E", name.split(GEMM_PANEL, 1)[1])
+        return int(ints[2]) if len(ints) >= 3 else None
     kern = GEMM if GEMM in name else GEMM_WS if GEMM_WS in name else None
     ints = re.findall(r"Li(\d+)E", name.split(kern, 1)[1]) if kern else []
     return int(ints[6]) if len(ints) >= 7 else None
