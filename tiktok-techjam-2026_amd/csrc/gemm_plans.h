@@ -11,15 +11,14 @@ enum { kStaged = 0, kDtl = 1, kWs = 2, kPanel = 3 };
 
 struct GemmPlan {
   int kind, bm, bn, wm, wn, bkb, stages;
-  double eff;       // prior used by auto_plan
+  double eff;       // prior of auto_plan's fall-back
   int ksplit = 1;   // K groups per workgroup (direct-to-LDS kernel)
   int loaders = 0;  // DMA-only waves (wave-specialized kernel)
 };
 
-// 2-byte types (bf16/fp16), BK = 64.  Measured on MI355X (bf16, C4/C5
-// projections): the 64x64-wave-tile plan 7 is best while there are too few
-// 256x256 tiles to fill two rounds of the 256 CUs, the 8-wave 256x256 plan 8
-// beyond that.  (A 4-stage ring of 64-byte rows was tried and dropped: it
+// 2-byte types (bf16/fp16), BK = 64.  Which one a launch takes by default is
+// gemm.hip's estimate (kAuto16); `eff` only ranks the plans where no estimated
+// tile's offsets reach the rows.  (A 4-stage ring of 64-byte rows was tried and dropped: it
 // measured 50% LDS bank-conflict cycles and no gain.)
 static const GemmPlan kPlans16[] = {
     {kStaged, 256, 256, 2, 2, 128, 2, 0.50},  // 0
