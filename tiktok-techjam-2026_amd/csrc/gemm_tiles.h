@@ -836,6 +836,31 @@ __device__ __forceinline__ void lds_dma16(u32x4 rsrc, uint32_t voff, uint32_t ld
   asm volatile("buffer_load_dwordx4 %0, %1, 0 offen lds" ::"v"(voff), "s"(rsrc), "{m0}"(lds_addr));
 }
 
+// Waits until panel_accumulate's MFMAs have written their results.  The
+// compiler does not see an MFMA in inline asm: it neither inserts the wait
+// states before another instruction may read the result (8 for a 4-pass MFMA
+// on gfx950) nor keeps a copy of an accumulator behind a wait that does not
+// name it.  So the waits here have the accumulators that they guard as
+// operands, those of the last step (A panel 1 x W panel 1); the others have that
+// step's 8 or more MFMAs behind them and pass through an empty asm, which ends
+// the main loop's registers here (without it the 256 x 256 tiles copied and
+// spilled accumulators between the loop and the wait).
+template <int FM, int FN> __device__ __forceinline__ void acc_written(Acc16<FM, FN>& acc) {
+  typedef PanelGeom<FM, FN> G;
+  constexpr int I1 = 2 * G::F[kPanelW0], J1 = 2 * G::F[kPanelA0];
+  __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+  for (int i = I1; i < 2 * FN; ++i)
+#pragma unroll
+    for (int j = J1; j < 2 * FM; j += 2) asm volatile("s_nop 7\n\ts_nop 1" : "+a"(acc[i][j]), "+a"(acc[i][j + 1]));
+#pragma unroll
+  for (int i = 0; i < 2 * FN; ++i)
+#pragma unroll
+    for (int j = 0; j < 2 * FM; j += 2)
+      if (i < I1 || j < J1) asm volatile("" : "+a"(acc[i][j]), "+a"(acc[i][j + 1]));
+  __builtin_amdgcn_sched_barrier(0);
+}
+
 // acc += A[m0 : m0 + 64 FM, :] W[n0 : n0 + 64 FN, :]^T for this wave's
 // sub-tile.  On return every DMA has landed and the workgroup has met at a
 // barrier, so the LDS ring may be reused.
@@ -953,7 +978,8 @@ __device__ __forceinline__ void panel_accumulate(char* smem, const T* __restrict
   asm volatile("s_barrier" ::: "memory");
   __builtin_amdgcn_sched_barrier(0);
   const int nkt = (int)((kend + 127u) / 128u);
-  for (int t = 0; t < nkt; t += 2) {
+  int t = 0;
+  do {  // (K = 0: one trip over zeros)
     step(c0, c0, W1, c0, W0, c0, t + 2, A1);
     step(c0, c1, A1, c0, W1, c0, t + 2, A0);
     step(c1, c1, A0, c1, A1, c0, t + 2, W1);
@@ -962,11 +988,10 @@ __device__ __forceinline__ void panel_accumulate(char* smem, const T* __restrict
     step(c0, c0, A1, c1, W0, c1, t + 3, A0);
     step(c1, c0, A0, c0, A1, c1, t + 3, W0);
     step(c1, c1, W0, c0, A0, c0, t + 4, W1);
-  }
+  } while ((t += 2) < nkt);
+  acc_written<FM, FN>(acc);
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
   __syncthreads();
-  // the last MFMAs' results, which the compiler does not track, are written
-  asm volatile("s_nop 15\n\ts_nop 15" ::: "memory");
 }
 
 template <typename T, int FM, int FN>
