@@ -259,6 +259,29 @@ def test_gemm_default_tile_takes_any_k(device, dt, m, n, k):
     _close(res, (ref + r0.to(device).double()).cpu(), 2e-5, 1e-4)
 
 
+@pytest.mark.parametrize("rows,k,plan", [
+    (64, 72, -1), (64, 64, 9), (64, 192, 22),
+    (128, 64, 35), (128, 192, 35),  # odd counts of K tiles: the panel ring runs one more
+    (32, 2056, -1), (32, 2048, 26),
+])
+def test_gemm_pitch_at_the_offset_limit(device, rows, k, plan):
+    """Rows so far apart that a tile of `rows` of them ends within the last
+    64 KB of the 31-bit range: pieces past K must still arrive as zeros.  All
+    of the buffer but the operands is NaN."""
+    ld = (2 ** 31 - 1) // (rows * 2) // 8 * 8
+    assert rows * ld * 2 > 0x7fff0000
+    g = _gen(rows + k)
+    buf = torch.full((rows + 1, ld), float("nan"), dtype=torch.bfloat16, device=device)
+    a, w = buf[:rows, :k], buf[:rows, 4096:4096 + k]
+    a.copy_(torch.randn(rows, k, generator=g))
+    w.copy_(torch.randn(rows, k, generator=g) / math.sqrt(k))
+    ref = a.double() @ w.double().t()
+    out = ops.gemm(a, w, None, torch.full((rows, rows), float("nan"), dtype=torch.bfloat16, device=device),
+                   ops.EPI_BIAS, plan)
+    torch.cuda.synchronize()
+    _close(out, ref.cpu(), OUT_RTOL[torch.bfloat16], 1e-4)
+
+
 @pytest.mark.parametrize("m,n,k", [  # K past whole 32-deep tiles; the tile the default rule takes:
     (1, 4, 4), (700, 1028, 200),         # 64 x 64
     (130, 68, 260), (33, 1000, 2052),    # 32 x 32, K split in 4

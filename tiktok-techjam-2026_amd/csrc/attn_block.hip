@@ -147,7 +147,7 @@ __global__ __launch_bounds__(256) void attn_block_kernel(
   constexpr int NK = D / 64;  // K chunks
   auto dma = [&](int kt, int q) {
     char* sb = smem + (kt % kAbStages) * kAbStage;
-    const uint32_t kb = kt < NK ? (uint32_t)(kt * kAbBkb) : (uint32_t)kPastEnd;
+    const uint32_t kb = kt < NK ? (uint32_t)(kt * kAbBkb) : kPastEnd;
     if (q < kAbDA)
       __builtin_amdgcn_raw_ptr_buffer_load_lds(rsa, (lds_void*)(sb + (q * 4 + wave) * 1024), 16, voff[q] + kb,
                                                0, 0, 0);
@@ -177,7 +177,7 @@ __global__ __launch_bounds__(256) void attn_block_kernel(
         (void*)(bqkv != nullptr ? bqkv : wqkv), (short)0, bqkv != nullptr ? 3 * D * (int)sizeof(T) : 0, 0x00020000);
     const int seg = lane / 8;
     const uint32_t off = seg < 3 ? (uint32_t)((seg * D + kAbHd * h) * (int)sizeof(T) + (lane % 8) * 16)
-                                 : (uint32_t)kPastEnd;
+                                 : kPastEnd;
     __builtin_amdgcn_raw_ptr_buffer_load_lds(rsb, (lds_void*)(smem + Lay::BQKV_OFF), 16, off, 0, 0, 0);
   } else if (wave == 1 && h == 0 && bout != nullptr) {
     const __amdgpu_buffer_rsrc_t rso = __builtin_amdgcn_make_buffer_rsrc(

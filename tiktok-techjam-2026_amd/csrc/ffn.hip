@@ -42,6 +42,7 @@
 namespace tjk {
 
 constexpr int kFfnRows = 32;  // rows per workgroup
+constexpr int64_t kMaxWeightBytes = 0x7fff0000;  // limit of a weight (one buffer descriptor)
 constexpr int kFfnWaves = 4;
 
 // Physical 16-byte chunk of logical chunk c in row r of a resident operand
@@ -122,7 +123,7 @@ struct WStream {
 
   __device__ __forceinline__ void dma(int kt, int q) {
     char* sb = ring + (kt % STAGES) * STAGE;
-    const uint32_t kb = kt < nk ? (uint32_t)(kt * BKB) : (uint32_t)kPastEnd;
+    const uint32_t kb = kt < nk ? (uint32_t)(kt * BKB) : kPastEnd;
     __builtin_amdgcn_raw_ptr_buffer_load_lds(rsw, (lds_void*)(sb + (q * NW + wave) * 1024), 16,
                                              (uint32_t)(voff[q] + kb), 0, 0, 0);
   }
@@ -639,7 +640,7 @@ extern "C" int tjk_ffn(const void* a, int a_dtype, int64_t lda, const float* ln_
     return fail(TJK_EUNSUPPORTED, "tjk_ffn: unsupported d=%lld f=%lld splits=%d dtype=%d (f / splits must be 64 or "
                 "128; d in {128, 256, 512}, fp32 d <= 256)", (long long)d, (long long)f, splits, dtype);
   if (rows == 0) return TJK_OK;
-  if (rows > INT32_MAX / 2 || f > INT32_MAX || d * f * dtype_size(dtype) >= kPastEnd)
+  if (rows > INT32_MAX / 2 || f > INT32_MAX || d * f * dtype_size(dtype) >= kMaxWeightBytes)
     return fail(TJK_EUNSUPPORTED, "tjk_ffn: shape exceeds the 32-bit buffer range");
   if (!a || !w1 || !w2 || !out) return fail(TJK_EINVAL, "tjk_ffn: null pointer");
   const bool ln = ln_gamma != nullptr;
@@ -689,7 +690,7 @@ extern "C" int tjk_gemm_ln(const float* res, int64_t ld_res, const float* gamma,
     return fail(TJK_EINVAL, "tjk_gemm_ln: plan %d out of range [-1,%d)", plan_id, kLnGemmPlans);
   if (m == 0 || n == 0) return TJK_OK;
   if (!res || !gamma || !beta || !w || !c) return fail(TJK_EINVAL, "tjk_gemm_ln: null pointer");
-  if (m > INT32_MAX / 2 || n > INT32_MAX || n * ldw * dtype_size(dtype) >= kPastEnd)
+  if (m > INT32_MAX / 2 || n > INT32_MAX || n * ldw * dtype_size(dtype) >= kMaxWeightBytes)
     return fail(TJK_EUNSUPPORTED, "tjk_gemm_ln: shape exceeds the 32-bit buffer range");
   if (n % 4) return fail(TJK_EUNSUPPORTED, "tjk_gemm_ln: n=%lld must be a multiple of 4", (long long)n);
   const int es = dtype_size(dtype);

@@ -279,7 +279,7 @@ __global__ __launch_bounds__((WM * WN + L) * 64) void gemm_ws_kernel(
     auto dma = [&](int t, int q) {
       char* sb = smem + (t % STAGES) * STAGE;
       const int base = (q * L + lw) * G::RPI;  // wave-uniform
-      const uint32_t kb = (uint32_t)(t * BKB) + lcb < kend ? (uint32_t)(t * BKB) : (uint32_t)kPastEnd;
+      const uint32_t kb = (uint32_t)(t * BKB) + lcb < kend ? (uint32_t)(t * BKB) : kPastEnd;
       if (base < BM) {
         const int r = base + lane / G::CPR;
         __builtin_amdgcn_raw_ptr_buffer_load_lds(

@@ -521,8 +521,10 @@ template <> __device__ __forceinline__ int swz<64>(int r) { return ((r >> 1) ^ (
 
 typedef __attribute__((address_space(3))) void lds_void;
 
-// Byte offset that lies beyond any buffer descriptor range used here.
-constexpr int kPastEnd = 0x7fff0000;
+// Byte offset beyond any buffer descriptor range (those are signed 32-bit
+// counts); a row's offset inside a range added to it still fits 32 bits.
+constexpr uint32_t kPastEnd = 0x80000000u;
+static_assert(kPastEnd > (uint32_t)INT32_MAX, "pieces past K must lie outside every range");
 
 // Tile geometry shared by the direct-to-LDS kernels.
 template <typename T, int BM, int BN, int WM, int WN, int BKB, int STAGES, int KSPLIT>
@@ -623,7 +625,7 @@ __device__ __forceinline__ void dtl_accumulate(
   // into its slot; past K it points outside the range and moves nothing.
   auto k_off = [&](int it, int i) __attribute__((always_inline)) {
     const uint32_t kt = (uint32_t)((it * KSPLIT + kg) * BKB);
-    return kt + (NW == 1 && (i & 1) ? lcb ^ 16u : lcb) < kend ? kt : (uint32_t)kPastEnd;
+    return kt + (NW == 1 && (i & 1) ? lcb ^ 16u : lcb) < kend ? kt : kPastEnd;
   };
   auto dma1 = [&](int it, int q) {
     char* sb = gsm + (it % STAGES) * STAGE;
@@ -902,7 +904,7 @@ __device__ __forceinline__ void panel_accumulate(char* smem, const T* __restrict
   auto dma = [&](auto P, auto S, int kt, int i) __attribute__((always_inline)) {
     constexpr int p = decltype(P)::value, s = decltype(S)::value;
     const uint32_t kb = (uint32_t)kt * 128u;
-    const uint32_t ko = kb + lcb < kend ? kb : (uint32_t)kPastEnd;
+    const uint32_t ko = kb + lcb < kend ? kb : kPastEnd;
     const uint32_t v = p == kPanelA0 ? va0[i] : p == kPanelA1 ? va1[i] : p == kPanelW0 ? vw0[i] : vw1[i];
     lds_dma16(p < 2 ? rsa : rsw, v + ko, lds0 + s * G::SLOT + G::OFF[p] + (i * 4 + wave) * 1024);
   };
