@@ -156,6 +156,8 @@ int tjk_gemm_bias_residual_from(const void* a, int64_t lda, const void* w, int64
  * k_groups add up K in the same order: they give identical results. */
 int tjk_gemm_plan_count(int dtype);
 int tjk_gemm_plan_info(int dtype, int id, int* block_m, int* block_n, int* waves, int* k_groups);
+/* The plan that plan_id -1 takes for a shape, row pitches and epilogue (host only). */
+int tjk_gemm_default_plan(int64_t m, int64_t n, int64_t k, int64_t lda, int64_t ldw, int dtype, int epilogue);
 
 /*
  * Flash-attention forward over a packed QKV buffer laid out [B, S, 3, H, hd]

@@ -629,6 +629,35 @@ def test_rocprof_summary_labels_deferred_projections():
     assert rs._gemm_epilogue(ws4) == 4 and rs._relabel("gemm_out_residual", ws4) == "gemm_out_residual"
 
 
+@pytest.mark.parametrize("dt,ids", [(torch.float32, _lib.F32), (torch.bfloat16, _lib.BF16)])
+def test_default_gemm_plan_keeps_the_class_of_the_shape(dt, ids):
+    """The plan that -1 takes sums K as the tile timing's candidates for the
+    shape do (tiles.k_class), also where the rows are too far apart for the
+    larger tiles; the timing's candidates are whole-K-tile ones."""
+    import random
+    from tjkernels import ops, tiles
+    lib, rng = _lib.load(), random.Random(5)
+    groups = {p[0]: p[4] for p in ops.gemm_plans(dt)}
+    es = 4 if dt == torch.float32 else 2
+
+    def check(m, n, k, lda, ldw):
+        for epi in (_lib.EPI_BIAS, _lib.EPI_BIAS_RESIDUAL):
+            plan = lib.tjk_gemm_default_plan(m, n, k, lda, ldw, ids, epi)
+            assert groups[plan] == tiles.k_class((m + 63) // 64 * 64, n, k, dt), (m, n, k, lda, ldw, plan)
+
+    for _ in range(2000):
+        m, n = int(2 ** rng.uniform(0, 14)), 4 * int(2 ** rng.uniform(0, 11))
+        k = 128 // es * rng.randint(1, 64)
+        reach = (2 ** 31 - 1) // (64 * es) // 16 * 16  # rows that tiles of 64 of them still reach
+        if dt == torch.bfloat16 and -(-m // 128) * -(-n // 128) >= 128:
+            reach //= 2  # farther ones are refused
+        check(m, n, k, k, k)
+        check(m, n, k, rng.randint(k, reach) // 16 * 16, k)
+        check(m, n, k, k, rng.randint(k, reach) // 16 * 16)
+    if dt == torch.float32:
+        check(64, 64, 128, 3000000, 128)  # one K group: fewer than 256 of K
+
+
 def test_plan_tile_rows_round_trip_and_validation():
     """Plan.tile_rows (the row bucket the autotuner measured the gemm_*
     tiles at) survives plans.json and must be a row count >= 0."""

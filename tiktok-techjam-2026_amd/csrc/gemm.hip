@@ -113,7 +113,8 @@ static int least_estimate(const AutoTile (&table)[NT], const GemmPlan* p, int64_
 // any K here: pieces of the last K tile past K arrive as zeros.  (A plan asked
 // for by id takes whole K tiles only.)  Rows too far apart for those tiles'
 // 31-bit offsets go by the least (full-chip rounds of 256 workgroups) x (tile
-// area / prior) over the plans that take the K: staged, or refused.
+// area / prior) over the plans with one K group that take the K: staged, or
+// refused; fp32 ones of class 4 take its tile as far as 64 x 64 tiles reach.
 template <typename T>
 static int auto_plan(int64_t M, int64_t N, int64_t K, int64_t lda, int64_t ldw, int epi) {
   int count;
@@ -123,13 +124,14 @@ static int auto_plan(int64_t M, int64_t N, int64_t K, int64_t lda, int64_t ldw, 
     if (K % 64 == 0 && !span_ok(p[narrow], lda, ldw, sizeof(T))) return narrow;
     const int best = least_estimate<T>(kAuto16, p, M, N, K, lda, ldw, epi);
     if (best >= 0) return best;
-  } else if (span_ok(p[3], lda, ldw, sizeof(T))) {
-    return least_estimate<T>(kAuto32, p, M, N, K, lda, ldw, epi);
+  } else {
+    if (span_ok(p[3], lda, ldw, sizeof(T))) return least_estimate<T>(kAuto32, p, M, N, K, lda, ldw, epi);
+    if (k_class<T>(M, N, K) == 4 && span_ok(p[4], lda, ldw, sizeof(T))) return 5;
   }
   int best = 0;
   double best_cost = 1e300;
   for (int i = 0; i < count; ++i) {
-    if (p[i].kind != kStaged && !dtl_ok(p[i], K, lda, ldw, sizeof(T))) continue;
+    if (p[i].ksplit > 1 || (p[i].kind != kStaged && !dtl_ok(p[i], K, lda, ldw, sizeof(T)))) continue;
     const int64_t tiles = ((M + p[i].bm - 1) / p[i].bm) * ((N + p[i].bn - 1) / p[i].bn);
     const int64_t rounds = (tiles + 255) / 256;
     const double cost = (double)rounds * p[i].bm * p[i].bn / p[i].eff;
@@ -182,6 +184,17 @@ extern "C" int tjk_gemm_plan_info(int dtype, int id, int* block_m, int* block_n,
   if (waves) *waves = p[id].wm * p[id].wn * p[id].ksplit + p[id].loaders;
   if (k_groups) *k_groups = p[id].ksplit;
   return TJK_OK;
+}
+
+extern "C" int tjk_gemm_default_plan(int64_t m, int64_t n, int64_t k, int64_t lda, int64_t ldw, int dtype,
+                                     int epilogue) {
+  if (m <= 0 || n <= 0 || k < 0 || lda < k || ldw < k || m > INT32_MAX || n > INT32_MAX || k > INT32_MAX)
+    return fail(TJK_EINVAL, "tjk_gemm_default_plan: bad shape");
+  if (epilogue < TJK_EPI_BIAS || epilogue > TJK_EPI_BIAS_RESIDUAL)
+    return fail(TJK_EINVAL, "tjk_gemm_default_plan: bad epilogue %d", epilogue);
+  if (dtype == TJK_F32) return auto_plan<float>(m, n, k, lda, ldw, epilogue);
+  if (dtype == TJK_F16 || dtype == TJK_BF16) return auto_plan<bf16>(m, n, k, lda, ldw, epilogue);
+  return fail(TJK_EINVAL, "tjk_gemm_default_plan: bad dtype %d", dtype);
 }
 
 extern "C" int tjk_gemm_bias(const void* a, int64_t lda, const void* w, int64_t ldw,

@@ -99,7 +99,8 @@ static const GemmPlan kPlans32[] = {
     // leave most CUs idle (256 x 1024 x 1024 22.9 -> 9.4 us); 6: the tile
     // between 64 x 64 and 128 x 128 (5690 x 1024 x 1792 180 -> 168 us).
     {kDtl, 32, 32, 1, 1, 128, 2, 0.3, 4},    // 5 4 waves, 64 KB
-    {kDtl, 128, 64, 2, 2, 128, 2, 0.6},      // 6 wave tile 64x32
+    // (6's prior: never ahead of 2 in the fall-back)
+    {kDtl, 128, 64, 2, 2, 128, 2, 0.5},      // 6 wave tile 64x32
 };
 
 template <typename T>

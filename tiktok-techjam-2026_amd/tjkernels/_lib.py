@@ -39,6 +39,7 @@ _SIGNATURES = {
     "tjk_gemm_plan_count": (_i32, [_i32]),
     "tjk_gemm_plan_info": (_i32, [_i32, _i32, ctypes.POINTER(_i32), ctypes.POINTER(_i32),
                                   ctypes.POINTER(_i32), ctypes.POINTER(_i32)]),
+    "tjk_gemm_default_plan": (_i32, [_i64, _i64, _i64, _i64, _i64, _i32, _i32]),
     "tjk_flash_fwd": (_i32, [_vp, _i64, _i64, _i64, _i64, _vp, _i64, _i32, _i32, _i32, _i32,
                              _f32, _i32, _vp, _vp, _vp, _i32, _i32, _vp]),
     "tjk_flash_plan_count": (_i32, [_i32]),
