@@ -106,3 +106,33 @@ def test_panel_gemm_reads_results_after_their_wait(tmp_path, elem):
         assert sum(l.startswith("v_mfma") for l in code) >= 8, name
         assert not _early_uses(code), (name, _early_uses(code)[:3])
         assert not any(l.startswith("scratch_") for l in code), name
+
+
+OBJDUMP = shutil.which("llvm-objdump") or "/opt/rocm/llvm/bin/llvm-objdump"
+LIB = CSRC.parent / "tjkernels" / "libtjk.so"
+
+
+def _library_kernels(tmp_path, lib, what):
+    """(name, instructions) of the kernels named `what` in a built library."""
+    copy = tmp_path / "lib.so"
+    shutil.copy(lib, copy)
+    subprocess.run([OBJDUMP, "--offloading", str(copy)], check=True, capture_output=True, cwd=tmp_path)
+    for part in sorted(tmp_path.glob("lib.so.*gfx950*")):
+        text = subprocess.run([OBJDUMP, "-d", "--no-show-raw-insn", "--no-leading-addr", str(part)], check=True,
+                              capture_output=True, text=True).stdout
+        for m in re.finditer(r"^<(\S*" + what + r"\S*)>:\n((?:\t.*\n)+)", text, re.M):
+            yield m.group(1), [l.split("//")[0].strip() for l in m.group(2).splitlines()]
+
+
+@pytest.mark.skipif(not Path(OBJDUMP).exists() or not LIB.exists(), reason="needs llvm-objdump and the built library")
+def test_unmasked_attention_copies_before_it_waits(tmp_path):
+    """The K / V copies of a workgroup's first tiles go out before anything
+    waits for a load (of Q: a memory round trip more per workgroup)."""
+    seen = 0
+    for name, code in _library_kernels(tmp_path, LIB, "flash_pipe_kernelI"):
+        if re.search(r"ELi[05]ELi[48]EEE", name) is None:  # no mask: kMaskNone, kMaskNoneFull; 4 or 8 waves
+            continue
+        seen += 1
+        first = next(i for i, l in enumerate(code) if l.startswith("buffer_load") and l.endswith("lds"))
+        assert not any("vmcnt" in l for l in code[:first]), name
+    assert seen >= 20, seen

@@ -574,9 +574,10 @@ __device__ __forceinline__ void fa_lds_dma16(u32x4 rsrc, uint32_t voff, uint32_t
 // rows) and 96 (128 columns computed) before: 4 x 2048 x 16 heads, bf16
 // causal, 40.0 -> 37.4 us at 32, 77.8 -> 65.9 at 96; with a key mask 72 -> 41
 // and 212 -> 62.
-// kMaskBytesFull: kMaskBytes with head_dim == HDC.  kMaskNoneRegs: no mask,
-// head_dim == HDC, tiles through registers (see launch_pipe).
-enum { kMaskNone = 0, kMaskList = 1, kMaskBytes = 2, kMaskBytesFull = 3, kMaskNoneRegs = 4 };
+// kMaskBytesFull, kMaskNoneFull: kMaskBytes, kMaskNone with head_dim == HDC.
+// kMaskNoneRegs: no mask, head_dim == HDC, tiles through registers (see
+// launch_pipe).
+enum { kMaskNone = 0, kMaskList = 1, kMaskBytes = 2, kMaskBytesFull = 3, kMaskNoneRegs = 4, kMaskNoneFull = 5 };
 
 template <typename T, int HDP, int HDC, int MASK, int NW>
 __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(HDP <= 64 || NW == 8 ? 2 : 1, HDP <= 64 || NW == 8 ? 2 : 1))) void flash_pipe_kernel(
@@ -603,7 +604,7 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(HDP <= 
   // transposing ds_read_b64_tr_b16.  Otherwise (a key mask that is not listed,
   // small launches at head_dim 32) tiles pass through registers, V stored
   // transposed.
-  constexpr bool FULLHD = MASK == kMaskBytesFull || MASK == kMaskNoneRegs;
+  constexpr bool FULLHD = MASK == kMaskBytesFull || MASK == kMaskNoneRegs || MASK == kMaskNoneFull;
   constexpr bool KEYMASK = MASK == kMaskBytes || MASK == kMaskBytesFull, DMA = !KEYMASK && MASK != kMaskNoneRegs;
   static_assert(!DMA || HDP >= 64, "rows of whole 8-chunk XOR groups");
   // LIST (a key mask): the workgroup lists its admissible keys
@@ -642,6 +643,10 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(HDP <= 
     s_flag = &flag;
   }
 
+  // The epilogue's arguments are read here: a scalar load in flight during the
+  // tiles makes every wait for some of the LDS reads a wait for all of them
+  // (tiles through registers, 4 x 700 x 8 heads of 32: 9.73 -> 9.55 us).
+  if constexpr (MASK == kMaskNoneRegs) asm volatile("" ::"s"(out), "s"(ld_out));
   const int BH = B * H;
   // One work item: query block qb of (b, h) = bh over key tiles [t_lo,
   // t_hi).  slot -1: a whole item; slot s >= 0: the first half of a
@@ -731,30 +736,45 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(HDP <= 
   const int nkt = (kend + BNK - 1) / BNK;
   t_hi = min(t_hi, nkt);
 
-  // Q fragments (B operand of S^T): lane holds Q[q][16c + 8*hi + 0..7]
-  typename Mfma<T>::frag qf[KC];
-  {
-    const int q = wq0 + l32;
-    float z[8] = {0, 0, 0, 0, 0, 0, 0, 0};
-#pragma unroll
-    for (int c = 0; c < KC; ++c) qf[c] = Mfma<T>::pack(z);
-    if (FULLHD || hd == HDC) {  // all loads under one branch
-      if (q < Sb)
-#pragma unroll
-        for (int c = 0; c < KC; ++c) qf[c] = Mfma<T>::load(qbase + (int64_t)q * ss + 16 * c + 8 * hi);
-    } else {
-#pragma unroll
-      for (int c = 0; c < KC; ++c)
-        if (q < Sb && 16 * c + 8 * hi < hd) qf[c] = Mfma<T>::load(qbase + (int64_t)q * ss + 16 * c + 8 * hi);
-    }
-  }
-
   // K / V rows of this (b, h): the span from key 0 to the end of key Sb-1.
   // Tile t is read through a descriptor starting at its first key (scalar
   // work), so the per-lane offsets stay fixed across tiles; a tile past the
   // item's range gets an empty descriptor and reads as zeros.
   const uint32_t row_bytes = (uint32_t)(ss * (int64_t)sizeof(T));
   const int span = (int)(((int64_t)(Sb - 1) * ss + hd) * (int64_t)sizeof(T));
+
+  // Q fragments (B operand of S^T): lane holds Q[q][16c + 8*hi + 0..7], read
+  // through a descriptor over the same span of Q, rows and columns past the end
+  // from outside it (zeros): loads under a per-launch condition on head_dim were
+  // waited for ahead of the first K / V copies (8 x 1024 x 12 heads of 64, bf16
+  // causal, 28.4 us so, 27.5 now).  A whole head_dim of 128 (8 fragments, one
+  // workgroup per CU) and tiles through registers load each under the lane's
+  // condition, which waits for nothing (1 x 332 x 2 heads of 128 14.3 us, 14.7
+  // through the descriptor; masked 8 x 192 x 12 of 128 12.4 and 12.5; 1 x 1019 x
+  // 4 heads of 64 14.1 and 13.9).
+  constexpr uint32_t kPastRange = 0x80000000u;  // beyond any descriptor's range
+  typename Mfma<T>::frag qf[KC];
+  {
+    const int q = wq0 + l32;
+    const __amdgpu_buffer_rsrc_t rsq = __builtin_amdgcn_make_buffer_rsrc((void*)qbase, (short)0, span, 0x00020000);
+#pragma unroll
+    for (int c = 0; c < KC; ++c) {
+      const int col = 16 * c + 8 * hi;
+      if constexpr (!DMA || (FULLHD && HDP != 64)) {
+        if (q < Sb && (FULLHD || col < hd)) {
+          qf[c] = Mfma<T>::load(qbase + (int64_t)q * ss + col);
+        } else {
+          float z[8] = {0, 0, 0, 0, 0, 0, 0, 0};
+          qf[c] = Mfma<T>::pack(z);
+        }
+      } else {
+        const uint32_t off =
+            q < Sb && (FULLHD || col < hd) ? (uint32_t)q * row_bytes + (uint32_t)(2 * col) : kPastRange;
+        qf[c] = __builtin_bit_cast(typename Mfma<T>::frag, __builtin_amdgcn_raw_buffer_load_b128(rsq, off, 0, 0));
+      }
+    }
+  }
+
   uint4 rk[KPT], rv0[VPT], rv1[VPT];
   auto load_kv_into = [&](int t, uint4 (&rk)[KPT], uint4 (&rv0)[VPT], uint4 (&rv1)[VPT]) __attribute__((always_inline)) {
     const int64_t t_elems = (int64_t)t * BNK * ss;
@@ -828,14 +848,13 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(HDP <= 
     const int r0 = r & 1, r1 = (r >> 1) & 1, r2 = (r >> 2) & 1, r3 = (r >> 3) & 1;
     return CPR == 8 ? (r1 | (r3 << 1) | ((r1 ^ r2) << 2)) : (r0 | (r1 << 1) | ((r0 ^ r2) << 2) | ((r1 ^ r3) << 3));
   };
-  constexpr uint32_t kPastRange = 0x80000000u;  // beyond any descriptor's range: zeros
   uint32_t dvoff[NDK];
   const uint32_t lds_ring = (uint32_t)(uintptr_t)(lds_void*)smem;
 #pragma unroll
   for (int q = 0; q < NDK; ++q) {
     const int r = (q * NW + wave) * RPI + lane / CPR;
     const int c = (lane % CPR) ^ swz(r);
-    dvoff[q] = (LIST ? 0 : (uint32_t)r * row_bytes) + (c * VEC < hd ? (uint32_t)(c << 4) : kPastRange);
+    dvoff[q] = (LIST ? 0 : (uint32_t)r * row_bytes) + (FULLHD || c * VEC < hd ? (uint32_t)(c << 4) : kPastRange);
   }
   // LIST: this lane's listed key of each DMA instruction of the tile that is
   // copied next, read from the list one tile ahead
@@ -1384,7 +1403,7 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(HDP <= 
   // MiB or more can write them through the L2 (its 8-byte pieces 2 KB apart,
   // stored straight from the accumulator layout, measured 4 us slower per C4
   // launch written through, one by one).  Needs 16-byte aligned rows.
-  const bool staged = DMA && hd == HDC && ((uintptr_t)out & 15) == 0 && (ld_out % 8) == 0;
+  const bool staged = DMA && (FULLHD || hd == HDC) && ((uintptr_t)out & 15) == 0 && (ld_out % 8) == 0;
   if (staged) {
     // The ring is free once every wave's copies have landed (the copies of
     // tiles past the item write zeros too) and every wave is past its last
@@ -1455,7 +1474,7 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(HDP <= 
   // cannot be placed: it is counted in the error word and dropped.  A slot
   // outside [0, n_slots) (or its second-half image) has no partial to
   // publish or merge: the item's rows are written as NaN and counted.
-  if (MASK == kMaskNone && NW == 4 && work != nullptr) {
+  if ((MASK == kMaskNone || MASK == kMaskNoneFull) && NW == 4 && work != nullptr) {
     for (int j = blockIdx.x; j < n_work; j += gridDim.x) {
       const int4 it = work[j];
       if (it.x == -1) continue;
@@ -1495,10 +1514,13 @@ static int launch_sched(const void* qkv, int64_t ss, int64_t sc, int64_t sh, voi
     // a fill kernel, not hipMemsetAsync: the call may be recorded into a graph
     hipLaunchKernelGGL(clear_words_kernel, dim3(1), dim3(256), 0, st, flags - 1, n_slots + 1);
   }
-  hipLaunchKernelGGL((flash_pipe_kernel<T, HDP, HDC, kMaskNone, 4>), dim3((unsigned)n_lists), dim3(256), 0, st,
-                     (const T*)qkv, (int64_t)0, ss, sc, sh, (T*)out, ld_out, B, S, H, hd, scale_log2, causal,
-                     (const int32_t*)nullptr, (const uint8_t*)nullptr, cu_seqlens, 0,
-                     reinterpret_cast<const int4*>(work), n_work, partials, flags, n_slots, 1);
+#define TJK_PIPE_SCHED(KM)                                                                                         \
+  hipLaunchKernelGGL((flash_pipe_kernel<T, HDP, HDC, KM, 4>), dim3((unsigned)n_lists), dim3(256), 0, st,           \
+                     (const T*)qkv, (int64_t)0, ss, sc, sh, (T*)out, ld_out, B, S, H, hd, scale_log2, causal,      \
+                     (const int32_t*)nullptr, (const uint8_t*)nullptr, cu_seqlens, 0,                              \
+                     reinterpret_cast<const int4*>(work), n_work, partials, flags, n_slots, 1)
+  if (hd == HDC) TJK_PIPE_SCHED(kMaskNoneFull); else TJK_PIPE_SCHED(kMaskNone);
+#undef TJK_PIPE_SCHED
   return check_launch("tjk_flash_fwd_sched");
 }
 
@@ -1552,7 +1574,7 @@ static int launch_pipe(const void* qkv, int64_t sb, int64_t ss, int64_t sc, int6
         return check_launch("tjk_flash_fwd");
       }
     }
-    TJK_PIPE(HDP, HDC, kMaskNone, NW8);
+    if (hd == HDC) TJK_PIPE(HDP, HDC, kMaskNoneFull, NW8); else TJK_PIPE(HDP, HDC, kMaskNone, NW8);
   }
 #undef TJK_PIPE
   return check_launch("tjk_flash_fwd");
@@ -1868,7 +1890,7 @@ extern "C" int tjk_flash_sched_occupancy(int head_dim, int dtype) {
   hipError_t e = hipErrorInvalidValue;
   const bool h16 = dtype == TJK_F16;
 #define TJK_OCC(TT, HDP, HDC) \
-  e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&blocks, flash_pipe_kernel<TT, HDP, HDC, kMaskNone, 4>, 256, 0)
+  e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&blocks, flash_pipe_kernel<TT, HDP, HDC, kMaskNoneFull, 4>, 256, 0)
   if (head_dim <= 32) { if (h16) TJK_OCC(f16, 64, 32); else TJK_OCC(bf16, 64, 32); }
   else if (head_dim <= 64) { if (h16) TJK_OCC(f16, 64, 64); else TJK_OCC(bf16, 64, 64); }
   else if (head_dim <= 96) { if (h16) TJK_OCC(f16, 128, 96); else TJK_OCC(bf16, 128, 96); }
