@@ -658,6 +658,22 @@ def test_default_gemm_plan_keeps_the_class_of_the_shape(dt, ids):
         check(64, 64, 128, 3000000, 128)  # one K group: fewer than 256 of K
 
 
+@pytest.mark.parametrize("m,n,k,epi,good", [  # plans timed within 3% of the fixed rule of before the estimates, or faster
+    (6459, 448, 832, 2, (7, 9)), (7139, 3968, 192, 0, (7, 8)), (7668, 1984, 192, 2, (7, 8, 9, 15, 33)),
+    (10146, 320, 704, 2, (7,)), (13388, 1536, 320, 1, (7, 35)), (2883, 1344, 320, 2, (7, 9, 15)),
+    (4075, 3520, 320, 2, (7, 8, 33)), (12910, 3008, 192, 2, (7, 8, 9, 15, 34)), (495, 5120, 1216, 0, (7, 35)),
+    (1223, 5184, 320, 2, (7,)), (540, 5632, 256, 2, (7, 9)), (10830, 640, 320, 2, (7,)),
+    (11798, 3712, 256, 2, (7, 8, 15, 34)), (6122, 7232, 192, 0, (8,)), (14378, 7616, 128, 2, (7, 8, 15, 34, 35)),
+    (5430, 3072, 1024, 0, (14,)), (5430, 4096, 1024, 1, (34,)), (8192, 8192, 2048, 1, (33,)),
+    (8192, 2048, 8192, 2, (33,)),
+])
+def test_default_gemm_plan_is_no_slower_than_the_fixed_rule(m, n, k, epi, good):
+    """Launches that an estimate without plans 7 and 8, and with an odd number
+    of K tiles in the panel rings, made 5-16% slower (profiles/gemm_tiles.csv),
+    and four that it speeds up."""
+    assert _lib.load().tjk_gemm_default_plan(m, n, k, k, k, _lib.BF16, epi) in good
+
+
 def test_plan_tile_rows_round_trip_and_validation():
     """Plan.tile_rows (the row bucket the autotuner measured the gemm_*
     tiles at) survives plans.json and must be a row count >= 0."""

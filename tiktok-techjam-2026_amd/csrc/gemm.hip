@@ -36,32 +36,38 @@ static int k_class(int64_t M, int64_t N, int64_t K) {
 // Estimated microseconds of a launch on MI355X: with `tiles`
 // workgroups, `per_cu` of them resident per CU, a launch is `rounds` fillings
 // of the chip, in which the fullest CU runs `load` workgroups in all, each of
-// `steps` K tiles (per K group), and stores `mb` MB of output (read and
-// written, for a residual):
+// `steps` K tiles (per K group; the panel ring runs an even number), and stores
+// `mb` MB of output (read and written, for a residual):
 //   c0 + c1 rounds + c2 rounds steps + c3 load + c4 load steps + c5 mb
-// (mb at 5 TB/s).  The coefficients are a non-negative least squares fit, by
-// relative error, over a sweep of 475 launches (16 to 16384 rows, widths 128 to
-// 8192, every epilogue) timed with every plan; each is within 4-11% on
-// average.  The tile the estimate picks is 0.7% slower than the best plan of
-// its class (geometric mean over the sweep); the fixed rule before it (8 from
-// two rounds of 256 x 256 tiles, 7 from 128 tiles of 128 x 128, else 9) was
-// 29% slower: 5430 x 3072 x 1024 47 us against 36, 128 x 512 x 2048 with the
-// residual 11.7 against 5.6.  fp32: 208 launches, each coefficient set within
-// 1.3-2.5% on average; 0.6% slower than the best plan, where the rule before
-// it (rounds x area / prior) was 58% slower (1284 x 1536 x 512 37 us against
-// 22.6, 128 x 512 x 512 12.6 against 6.4).
+// (mb at 5 TB/s).  The coefficients are a non-negative least squares fit by
+// relative error to launches timed with every plan; profiles/gemm_tiles.csv
+// holds the launches and gemm_tiles.md what the estimate loses on them.  One K
+// group: 2013 launches (16 to 16384 rows, widths and K up to 8192, every
+// epilogue), weighted towards plans near the best of their launch; the tile
+// picked is 0.3% slower than the best of the eight (geometric mean), and 9%
+// faster than the fixed rule before it (8 from 512 tiles of 256 x 256, 7 from
+// 128 of 128 x 128, else 9), 7 launches more than 2% slower, none 5%.  Without
+// 7, 8 and the panel ring's even steps it was 0.9% slower than the best and 32
+// launches more than 5% slower than that rule, most with K <= 384 and a
+// residual.  Two and four K groups: the best tile but for 4 of 1547 launches.
+// fp32: 0.5% slower than the best tile over 336 launches, none slower than the
+// rule before it (rounds x area / prior); K split in four, 364 launches, always
+// faster than any unsplit tile.
 struct AutoTile {
   int plan, per_cu;
   float c[6];
 };
 static const AutoTile kAuto16[] = {
-    // one K group: 64 x 64, 96 x 128, 192 x 128, 128 x 128, 256 x 256, 192 x 384
-    {9, 5, {1.259f, 1.086f, 0.174f, 0.489f, 0.134f, 0.351f}},
-    {15, 2, {0.000f, 3.318f, 0.183f, 0.403f, 0.250f, 0.563f}},
-    {34, 2, {0.796f, 5.075f, 0.019f, 0.362f, 0.505f, 0.604f}},
-    {35, 2, {0.043f, 4.829f, 0.048f, 0.071f, 0.344f, 0.476f}},
-    {33, 1, {0.000f, 0.000f, 0.983f, 11.714f, 0.000f, 0.896f}},
-    {14, 1, {0.000f, 0.000f, 1.163f, 9.811f, 0.000f, 1.307f}},
+    // one K group: 64 x 64, 96 x 128, panels 192 x 128, 128 x 128 and 256 x 256,
+    // 192 x 384, 128 x 128, 256 x 256
+    {9, 5, {1.954f, 0.733f, 0.089f, 0.411f, 0.163f, 0.362f}},
+    {15, 2, {0.980f, 1.220f, 0.379f, 1.098f, 0.185f, 0.442f}},
+    {34, 2, {1.536f, 2.753f, 0.131f, 0.924f, 0.505f, 0.498f}},
+    {35, 2, {1.513f, 2.455f, 0.129f, 0.170f, 0.347f, 0.652f}},
+    {33, 1, {0.000f, 0.000f, 1.323f, 8.871f, 0.000f, 0.575f}},
+    {14, 1, {0.000f, 0.000f, 1.638f, 7.071f, 0.000f, 0.726f}},
+    {7, 2, {1.595f, 1.016f, 0.289f, 1.104f, 0.318f, 0.529f}},
+    {8, 1, {0.000f, 0.000f, 1.499f, 5.760f, 0.000f, 0.625f}},
     // two K groups: 32 x 32, 32 x 64, 64 x 64, 128 x 64
     {25, 2, {1.108f, 1.764f, 0.151f, 0.325f, 0.073f, 0.000f}},
     {24, 1, {0.846f, 2.472f, 0.000f, 0.000f, 0.261f, 0.000f}},
@@ -91,7 +97,7 @@ static int least_estimate(const AutoTile (&table)[NT], const GemmPlan* p, int64_
   constexpr int BK = 128 / sizeof(T);
   const int cls = k_class<T>(M, N, K);
   const float mb = (float)M * (float)N * (epi_residual(epi) ? 8.f : (float)sizeof(T)) / 5e6f;
-  const float steps = (float)((K + BK - 1) / BK) / (float)cls;
+  const int64_t ktiles = (K + BK - 1) / BK;
   int best = -1;
   float best_us = 0.f;
   for (const AutoTile& t : table) {
@@ -100,6 +106,7 @@ static int least_estimate(const AutoTile (&table)[NT], const GemmPlan* p, int64_
     const int64_t tiles = ((M + q.bm - 1) / q.bm) * ((N + q.bn - 1) / q.bn), slots = 256 * t.per_cu;
     const int64_t full = tiles / slots, rest = tiles % slots;
     const float rounds = (float)(full + (rest > 0)), load = (float)(full * t.per_cu + (rest + 255) / 256);
+    const float steps = (float)(q.kind == kPanel ? ktiles + (ktiles & 1) : ktiles) / (float)cls;
     const float us = t.c[0] + rounds * (t.c[1] + t.c[2] * steps) + load * (t.c[3] + t.c[4] * steps) + t.c[5] * mb;
     if (best < 0 || us < best_us) {
       best = t.plan;
