@@ -225,21 +225,29 @@ def test_gemm_default_tile_keeps_its_class(device, m, n, k):
     assert torch.equal(outs[0], outs[1]) and torch.equal(outs[0], outs[2])
 
 
-@pytest.mark.parametrize("m,n,k", [  # the tile the default rule takes:
-    (1, 4, 8), (70, 68, 200),   # 64 x 64
-    (5547, 324, 40),            # 96 x 128
-    (5923, 1300, 72),           # 192 x 128, panel ring
-    (5467, 1036, 200),          # 128 x 128, panel ring
-    (5431, 2180, 520),          # 256 x 256, panel ring
-    (5430, 3072, 1000),         # 192 x 384
-    (33, 36, 1000),             # 32 x 32, K split in 2
-    (4161, 44, 520),            # 32 x 64, K split in 2
-    (2748, 164, 520),           # 64 x 64, K split in 2
-    (5534, 136, 600),           # 128 x 64, K split in 2
-    (33, 36, 2056), (4590, 40, 2600),  # 32 x 32, 32 x 64, K split in 4
+def _default_plan(a, w, epi):
+    from tjkernels import _lib
+    return _lib.load().tjk_gemm_default_plan(a.shape[0], w.shape[0], a.shape[1], a.stride(0), w.stride(0),
+                                             _lib.DTYPE_CODES[a.dtype], epi)
+
+
+@pytest.mark.parametrize("m,n,k,plain,residual", [  # the plans that the default rule takes
+    (1, 4, 8, 9, 9), (70, 68, 200, 9, 9),           # 64 x 64
+    (5547, 324, 40, 15, 15),                        # 96 x 128
+    (5923, 1300, 72, 34, 9), (5043, 1604, 80, 34, 34),  # 192 x 128, panel ring (2 K tiles)
+    (5467, 1036, 200, 35, 7), (2069, 1496, 464, 35, 35),  # 128 x 128, panel ring (4, 8 K tiles)
+    (6981, 416, 72, 7, 7),                          # 128 x 128
+    (5431, 2180, 520, 8, 8),                        # 256 x 256
+    (6637, 1988, 720, 8, 33), (8225, 1460, 1104, 33, 33),  # 256 x 256, panel ring (12, 18 K tiles)
+    (5430, 3072, 1000, 14, 34), (5441, 3020, 664, 14, 14),  # 192 x 384
+    (33, 36, 1000, 25, 25),                         # 32 x 32, K split in 2
+    (4161, 44, 520, 24, 24),                        # 32 x 64, K split in 2
+    (2748, 164, 520, 22, 22),                       # 64 x 64, K split in 2
+    (5534, 136, 600, 23, 23),                       # 128 x 64, K split in 2
+    (33, 36, 2056, 26, 26), (4590, 40, 2600, 27, 27),  # 32 x 32, 32 x 64, K split in 4
 ])
 @pytest.mark.parametrize("dt", [torch.bfloat16, torch.float16])
-def test_gemm_default_tile_takes_any_k(device, dt, m, n, k):
+def test_gemm_default_tile_takes_any_k(device, dt, m, n, k, plain, residual):
     """The default tile at K that is no multiple of 64, in every tile the rule
     takes: the columns between K and the rows' pitch are NaN and must not
     enter the sums (nor the rows past M and N, outside the buffers)."""
@@ -252,6 +260,7 @@ def test_gemm_default_tile_takes_any_k(device, dt, m, n, k):
     r0 = torch.randn(m, n, generator=g)
     ref = a[:, :k].to(device).double() @ w[:, :k].to(device).double().t() + b.to(device).double()
     ad, wd, bd = a.to(device)[:, :k], w.to(device)[:, :k], b.to(device)
+    assert [_default_plan(ad, wd, e) for e in (ops.EPI_BIAS, ops.EPI_BIAS_RESIDUAL)] == [plain, residual]
     out = ops.gemm(ad, wd, bd, torch.full((m, n), float("nan"), dtype=dt, device=device), ops.EPI_BIAS)
     res = ops.gemm(ad, wd, bd, r0.to(device), ops.EPI_BIAS_RESIDUAL)
     torch.cuda.synchronize()
@@ -282,15 +291,18 @@ def test_gemm_pitch_at_the_offset_limit(device, rows, k, plan):
     _close(out, ref.cpu(), OUT_RTOL[torch.bfloat16], 1e-4)
 
 
-@pytest.mark.parametrize("m,n,k", [  # K past whole 32-deep tiles; the tile the default rule takes:
-    (1, 4, 4), (700, 1028, 200),         # 64 x 64
-    (130, 68, 260), (33, 1000, 2052),    # 32 x 32, K split in 4
-    (700, 1024, 2052),                   # the last tile count that splits
-    (2050, 3068, 772),                   # 128 x 64
-    (4100, 4092, 68),                    # 128 x 128
+@pytest.mark.parametrize("m,n,k,plan", [  # K past whole 32-deep tiles; the plan that the default rule takes:
+    (1, 4, 4, 4), (700, 1028, 200, 4),               # 64 x 64
+    (130, 68, 260, 5), (33, 1000, 2052, 5),          # 32 x 32, K split in 4
+    (700, 1024, 2052, 5),                            # the last tile count that splits
+    (2050, 3068, 772, None), (4100, 4092, 68, None),  # 64 x 64 or, with the residual, 128 x 128
+    (1315, 3872, 68, 6),                             # 128 x 64
+    (2513, 2824, 36, 2),                             # 128 x 128
 ])
-def test_gemm_default_tile_fp32(device, m, n, k):
+def test_gemm_default_tile_fp32(device, m, n, k, plan):
+    a, w = torch.empty(m, k), torch.empty(n, k)
     for epi in (ops.EPI_BIAS, ops.EPI_BIAS_GELU, ops.EPI_BIAS_RESIDUAL):
+        assert _default_plan(a, w, epi) == (plan or (2 if epi == ops.EPI_BIAS_RESIDUAL else 4))
         _gemm_case(device, m, n, k, torch.float32, epi, -1)
 
 
