@@ -613,9 +613,9 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(HDP <= 
   // masked keys cost nothing.  Key limits (kend, lim, ...) then count listed
   // keys.  Before, every tile of a masked launch loaded 32 mask bytes per lane
   // and ran the unpipelined loop.  Measured with a quarter of the keys masked:
-  // 8 x 512 x 12 heads of 64, fp16, 27.6 -> 16.4 us (14.0 without a mask); 4 x
-  // 2048 x 16 heads of 64, bf16 causal, 109 (plan 1) -> 48 us (47); 2 x 4096 x
-  // 16 heads of 128, causal, 406 -> 114 us (137).
+  // 8 x 512 x 12 heads of 64, fp16, 29.4 -> 19.2 us (15.3 without a mask); 4 x
+  // 2048 x 16 heads of 64, bf16 causal, 109 (plan 1) -> 55 us (48); 2 x 4096 x
+  // 16 heads of 128, causal, 408 -> 122 us (132).
   constexpr bool LIST = MASK == kMaskList;
   constexpr int RB = HDP * (int)sizeof(T);  // DMA: bytes per K / V row
   constexpr int CPR = RB / 16, RPI = 64 / CPR, TILE_B = BNK * RB;
@@ -978,8 +978,14 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(HDP <= 
   // m_off: the exponent offset (log2 units) the running O and l are taken
   // relative to.  It is raised only when a query's scores exceed it by more
   // than kLazyRescale, so most tiles skip the O rescale; p <= 2^kLazyRescale
-  // is harmless in fp32 and in the 2-byte P.
-  constexpr float kLazyRescale = 8.0f;
+  // is harmless in fp32 and in the 2-byte P.  LIST: at every larger score, the
+  // running row max, so that a query's largest weight is exactly 1 in a 2-byte
+  // P, as in flash_fwd_kernel, which ran masked launches of 2048 keys and more
+  // before (error against 64 bits, bf16 causal 1 x 4096 x 2 heads of 64: 2.03e-3
+  // there, 2.08e-3 with the lazy offset, 2.02e-3 so; scores 4 times as spread
+  // 1.73, 1.86 and 1.73e-3).  It costs 8 x 512 x 12 heads of 64, fp16, 17.0 ->
+  // 18.5 us, 4 x 2048 x 16 causal 48 -> 54.
+  constexpr float kLazyRescale = LIST ? 0.f : 8.0f;
   float m_off = -INFINITY, l_run = 0.f;
 
   // softmax of one tile's scores (already masked) and O += V P
@@ -1076,7 +1082,7 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(HDP <= 
   // P = 2^(S * scale - m_off) packed to the MFMA type; returns this lane's
   // sum of the rounded P
   auto exp_pack = [&](const f32x16 (&sc)[2], Frag (&pf)[4]) __attribute__((always_inline)) -> float {
-    const float nb = -m_off;
+    const float nb = LIST && m_off == -INFINITY ? 0.f : -m_off;
     float l0 = 0.f, l1 = 0.f;
 #pragma unroll
     for (int stp = 0; stp < 4; ++stp) {
@@ -1160,6 +1166,20 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(HDP <= 
     }
     return lt;
   };
+  // LIST: raises the offset to the running row max before a tile's P
+  auto follow_max = [&](const f32x16 (&sc)[2]) __attribute__((always_inline)) {
+    const float mx = rowmax(sc);
+    if (__any(mx > m_off)) {
+      const float m_new = fmaxf(m_off, mx);
+      const float alpha = m_off == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(m_off - m_new);
+      l_run *= alpha;
+#pragma unroll
+      for (int hb = 0; hb < HB; ++hb)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) o[hb][r] *= alpha;
+      m_off = m_new;
+    }
+  };
   // accept P of tile `sc` (lane sum lt), or redo it from a raised offset
   auto settle = [&](const f32x16 (&sc)[2], Frag (&pf)[4], float lt) __attribute__((always_inline)) {
     if (__any(!(lt <= kSumLimit))) {
@@ -1232,7 +1252,7 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(HDP <= 
   int t = t_lo;
   // an unmasked first tile starts the offset at its row max, so the
   // interior loop does not redo it
-  if (t < n_int) m_off = rowmax(scur);
+  if (!LIST && t < n_int) m_off = rowmax(scur);
   f32x16 salt[2];
   Frag pf[4];
   // one interior step; j is tile t's ring slot (a constant in the unrolled loop)
@@ -1244,8 +1264,10 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(HDP <= 
       load_kv(tt + 3);
     }
     Frag vf[HB][4];
+    if constexpr (LIST) follow_max(sc);
     const float lt = qk_exp((j + 1) & (NST - 1), sn, sc, pf, j, vf);
-    settle(sc, pf, lt);
+    if constexpr (LIST) l_run += lt;
+    else settle(sc, pf, lt);
     pv(vf, pf, j);
     step_barrier();
   };
