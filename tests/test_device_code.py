@@ -124,15 +124,33 @@ def _library_kernels(tmp_path, lib, what):
             yield m.group(1), [l.split("//")[0].strip() for l in m.group(2).splitlines()]
 
 
-@pytest.mark.skipif(not Path(OBJDUMP).exists() or not LIB.exists(), reason="needs llvm-objdump and the built library")
-def test_unmasked_attention_copies_before_it_waits(tmp_path):
+@pytest.fixture(scope="module")
+def attention_rings(tmp_path_factory):
+    """{MASK: {name: instructions up to the first copy into LDS}} of the built
+    attention kernels whose K / V ring is filled by copies (4 or 8 waves)."""
+    if not Path(OBJDUMP).exists() or not LIB.exists():
+        pytest.skip("needs llvm-objdump and the built library")
+    rings = {}
+    for name, code in _library_kernels(tmp_path_factory.mktemp("lib"), LIB, "flash_pipe_kernelI"):
+        mask = int(re.search(r"ELi(\d)ELi[48]EEE", name).group(1))
+        first = [i for i, l in enumerate(code) if l.startswith("buffer_load") and l.endswith("lds")]
+        if first:
+            rings.setdefault(mask, {})[name] = code[:first[0]]
+    return rings
+
+
+def test_unmasked_attention_copies_before_it_waits(attention_rings):
     """The K / V copies of a workgroup's first tiles go out before anything
-    waits for a load (of Q: a memory round trip more per workgroup)."""
-    seen = 0
-    for name, code in _library_kernels(tmp_path, LIB, "flash_pipe_kernelI"):
-        if re.search(r"ELi[05]ELi[48]EEE", name) is None:  # no mask: kMaskNone, kMaskNoneFull; 4 or 8 waves
-            continue
-        seen += 1
-        first = next(i for i, l in enumerate(code) if l.startswith("buffer_load") and l.endswith("lds"))
-        assert not any("vmcnt" in l for l in code[:first]), name
-    assert seen >= 20, seen
+    waits for a load (of Q: a memory round trip more per workgroup).  Masks 0
+    and 5: kMaskNone, kMaskNoneFull."""
+    assert len(attention_rings[0]) >= 8 and len(attention_rings[5]) >= 8
+    for name, code in {**attention_rings[0], **attention_rings[5]}.items():
+        assert not any("vmcnt" in l for l in code), name
+
+
+def test_listed_attention_reads_eight_mask_blocks_at_a_time(attention_rings):
+    """kMaskList (1): eight mask reads go out before the first is waited for."""
+    assert len(attention_rings[1]) == 8
+    for name, code in attention_rings[1].items():
+        reads = [i for i, l in enumerate(code) if l.startswith("global_load_ubyte")]
+        assert len(reads) == 8 and not any("vmcnt" in l for l in code[reads[0]:reads[7]]), name

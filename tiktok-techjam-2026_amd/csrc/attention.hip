@@ -690,9 +690,11 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(HDP <= 
     const int nblk = (kend + 63) / 64;
     const uint8_t* const km = key_mask + (int64_t)b * S;
     for (int j0 = wave; j0 < 128; j0 += 8 * NW) {
-      uint8_t v[8];  // eight blocks' bytes in flight together
+      uint8_t v[8] = {};  // eight blocks' bytes in flight together: one condition for all of them
+      if (j0 < nblk) {
 #pragma unroll
-      for (int u = 0; u < 8; ++u) v[u] = j0 < nblk ? km[min((j0 + u * NW) * 64 + lane, S - 1)] : 0;
+        for (int u = 0; u < 8; ++u) v[u] = km[min((j0 + u * NW) * 64 + lane, S - 1)];
+      }
 #pragma unroll
       for (int u = 0; u < 8; ++u) {
         const uint64_t m = __ballot((j0 + u * NW) * 64 + lane < kend && v[u] != 0);
