@@ -656,8 +656,8 @@ def test_flash_head_dims(device, dt, hd, causal):
 @pytest.mark.parametrize("dt", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("seq", [129, 200, 515])
 def test_flash_head_dim_32_small_launches(device, seq, dt, causal):
-    """Head dim 32 up to 256 workgroups (tiles through registers) and above
-    (copied): the same bits, padded and with lengths, and both near fp64."""
+    """Head dim 32 on both sides of one 128-query workgroup per CU: the same
+    bits, padded and with lengths, and both near fp64."""
     heads, nqb = 4, (seq + 127) // 128
     small = 256 // (nqb * heads)
     g = _gen(seq)

@@ -570,14 +570,24 @@ __device__ __forceinline__ void fa_lds_dma16(u32x4 rsrc, uint32_t voff, uint32_t
 // HDP is the width of a K / V row in LDS, HDC the head-dim columns computed
 // (32, 64, 96 or 128 for head_dim up to that; HDP 64, 64, 128, 128).  Columns
 // of a row from head_dim on are copied from outside the buffer range: zeros.
-// Measured against the register-staged ring that served head_dim 32 (32-column
-// rows) and 96 (128 columns computed) before: 4 x 2048 x 16 heads, bf16
-// causal, 40.0 -> 37.4 us at 32, 77.8 -> 65.9 at 96; with a key mask 72 -> 41
-// and 212 -> 62.
+// Measured against the register-staged ring that served every head_dim but 64
+// and 128 before (128 columns computed at 96): 4 x 2048 x 16 heads of 96, bf16
+// causal, 77.8 -> 65.9 us, with a key mask 214 -> 63, of 32 with a key mask 72
+// -> 39.  Without one, head dims 8, 16 and 40 gain 0-11%, 72 to 96 11-17%; 24, 48
+// and 56 gain up to 11% and lose up to 13% (24) and 9% by the shape, 104 to 120
+// gain or lose 4%; head_dim 32 keeps its registers (PipeFull).
 // kMaskBytesFull, kMaskNoneFull: kMaskBytes, kMaskNone with head_dim == HDC.
-// kMaskNoneRegs: no mask, head_dim == HDC, tiles through registers (see
-// launch_pipe).
+// kMaskNoneRegs: no mask, head_dim == HDC, tiles through registers.
 enum { kMaskNone = 0, kMaskList = 1, kMaskBytes = 2, kMaskBytesFull = 3, kMaskNoneRegs = 4, kMaskNoneFull = 5 };
+
+// The unmasked variant of a whole head_dim HDC, and the width of its LDS rows.
+// Half of a 64-column row's copies are zeros at head_dim 32: its tiles pass
+// through registers in 32-column rows.  Registers / copies, us: 2 x 200 x 4 heads
+// bf16 causal 6.0 / 6.5, 4 x 700 x 8 9.5 / 9.8, 9 x 1119 x 12 32.8 / 36.6, 13 x
+// 1208 x 16 not causal 114 / 141, 6 x 4227 x 14 446 / 604; the copies' best was 8 x
+// 1024 x 12 causal, 24.2 / 23.5.  The same products and sums in the same order.
+template <int HDP, int HDC> struct PipeFull { static constexpr int MASK = kMaskNoneFull, WIDTH = HDP; };
+template <int HDP> struct PipeFull<HDP, 32> { static constexpr int MASK = kMaskNoneRegs, WIDTH = 32; };
 
 template <typename T, int HDP, int HDC, int MASK, int NW>
 __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(HDP <= 64 || NW == 8 ? 2 : 1, HDP <= 64 || NW == 8 ? 2 : 1))) void flash_pipe_kernel(
@@ -602,7 +612,7 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(HDP <= 
   // lds, K and V both key-major with 128- / 256-byte rows whose 16-byte chunks
   // are XOR-swizzled by row, and V^T fragments are gathered with the
   // transposing ds_read_b64_tr_b16.  Otherwise (a key mask that is not listed,
-  // small launches at head_dim 32) tiles pass through registers, V stored
+  // head_dim 32) tiles pass through registers, V stored
   // transposed.
   constexpr bool FULLHD = MASK == kMaskBytesFull || MASK == kMaskNoneRegs || MASK == kMaskNoneFull;
   constexpr bool KEYMASK = MASK == kMaskBytes || MASK == kMaskBytesFull, DMA = !KEYMASK && MASK != kMaskNoneRegs;
@@ -643,10 +653,6 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(HDP <= 
     s_flag = &flag;
   }
 
-  // The epilogue's arguments are read here: a scalar load in flight during the
-  // tiles makes every wait for some of the LDS reads a wait for all of them
-  // (tiles through registers, 4 x 700 x 8 heads of 32: 9.73 -> 9.55 us).
-  if constexpr (MASK == kMaskNoneRegs) asm volatile("" ::"s"(out), "s"(ld_out));
   const int BH = B * H;
   // One work item: query block qb of (b, h) = bh over key tiles [t_lo,
   // t_hi).  slot -1: a whole item; slot s >= 0: the first half of a
@@ -1498,7 +1504,7 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(HDP <= 
   // cannot be placed: it is counted in the error word and dropped.  A slot
   // outside [0, n_slots) (or its second-half image) has no partial to
   // publish or merge: the item's rows are written as NaN and counted.
-  if ((MASK == kMaskNone || MASK == kMaskNoneFull) && NW == 4 && work != nullptr) {
+  if (!KEYMASK && !LIST && NW == 4 && work != nullptr) {
     for (int j = blockIdx.x; j < n_work; j += gridDim.x) {
       const int4 it = work[j];
       if (it.x == -1) continue;
@@ -1538,12 +1544,13 @@ static int launch_sched(const void* qkv, int64_t ss, int64_t sc, int64_t sh, voi
     // a fill kernel, not hipMemsetAsync: the call may be recorded into a graph
     hipLaunchKernelGGL(clear_words_kernel, dim3(1), dim3(256), 0, st, flags - 1, n_slots + 1);
   }
-#define TJK_PIPE_SCHED(KM)                                                                                         \
-  hipLaunchKernelGGL((flash_pipe_kernel<T, HDP, HDC, KM, 4>), dim3((unsigned)n_lists), dim3(256), 0, st,           \
+#define TJK_PIPE_SCHED(HP, KM)                                                                                     \
+  hipLaunchKernelGGL((flash_pipe_kernel<T, HP, HDC, KM, 4>), dim3((unsigned)n_lists), dim3(256), 0, st,            \
                      (const T*)qkv, (int64_t)0, ss, sc, sh, (T*)out, ld_out, B, S, H, hd, scale_log2, causal,      \
                      (const int32_t*)nullptr, (const uint8_t*)nullptr, cu_seqlens, 0,                              \
                      reinterpret_cast<const int4*>(work), n_work, partials, flags, n_slots, 1)
-  if (hd == HDC) TJK_PIPE_SCHED(kMaskNoneFull); else TJK_PIPE_SCHED(kMaskNone);
+  typedef PipeFull<HDP, HDC> Full;
+  if (hd == HDC) TJK_PIPE_SCHED(Full::WIDTH, Full::MASK); else TJK_PIPE_SCHED(HDP, kMaskNone);
 #undef TJK_PIPE_SCHED
   return check_launch("tjk_flash_fwd_sched");
 }
@@ -1586,19 +1593,8 @@ static int launch_pipe(const void* qkv, int64_t sb, int64_t ss, int64_t sc, int6
   } else if (key_mask != nullptr) {
     TJK_PIPE(HDP, HDC, kMaskList, NW8);
   } else {
-    // head_dim 32 with at most one workgroup per CU: the latency of each tile
-    // counts, and half of a 64-column row's copies are zeros, so 32-column rows
-    // through registers are faster (bf16 causal, registers / copies: 2 x 200 x 4
-    // heads 6.2 / 6.5 us, 4 x 700 x 8 9.4 / 9.8, 2 x 1500 x 4 15.5 / 16.3); above
-    // that the copies are (16 x 160 x 12 1.02 times, 4 x 2048 x 16 40.0 / 37.4).
-    // The same products and sums in the same order either way.
-    if constexpr (HDC == 32) {
-      if (hd == 32 && nblk <= 256) {
-        TJK_PIPE(32, 32, kMaskNoneRegs, 4);
-        return check_launch("tjk_flash_fwd");
-      }
-    }
-    if (hd == HDC) TJK_PIPE(HDP, HDC, kMaskNoneFull, NW8); else TJK_PIPE(HDP, HDC, kMaskNone, NW8);
+    typedef PipeFull<HDP, HDC> Full;
+    if (hd == HDC) TJK_PIPE(Full::WIDTH, HDC, Full::MASK, NW8); else TJK_PIPE(HDP, HDC, kMaskNone, NW8);
   }
 #undef TJK_PIPE
   return check_launch("tjk_flash_fwd");
@@ -1913,12 +1909,15 @@ extern "C" int tjk_flash_sched_occupancy(int head_dim, int dtype) {
   int blocks = 0;
   hipError_t e = hipErrorInvalidValue;
   const bool h16 = dtype == TJK_F16;
-#define TJK_OCC(TT, HDP, HDC) \
-  e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&blocks, flash_pipe_kernel<TT, HDP, HDC, kMaskNoneFull, 4>, 256, 0)
-  if (head_dim <= 32) { if (h16) TJK_OCC(f16, 64, 32); else TJK_OCC(bf16, 64, 32); }
-  else if (head_dim <= 64) { if (h16) TJK_OCC(f16, 64, 64); else TJK_OCC(bf16, 64, 64); }
-  else if (head_dim <= 96) { if (h16) TJK_OCC(f16, 128, 96); else TJK_OCC(bf16, 128, 96); }
-  else { if (h16) TJK_OCC(f16, 128, 128); else TJK_OCC(bf16, 128, 128); }
+  // (the variants of a whole head_dim and of a part of it take the same rings,
+  // but for head_dim 32)
+#define TJK_OCC(TT, HDP, HDC, KM) \
+  e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&blocks, flash_pipe_kernel<TT, HDP, HDC, KM, 4>, 256, 0)
+  if (head_dim == 32) { if (h16) TJK_OCC(f16, 32, 32, kMaskNoneRegs); else TJK_OCC(bf16, 32, 32, kMaskNoneRegs); }
+  else if (head_dim < 32) { if (h16) TJK_OCC(f16, 64, 32, kMaskNone); else TJK_OCC(bf16, 64, 32, kMaskNone); }
+  else if (head_dim <= 64) { if (h16) TJK_OCC(f16, 64, 64, kMaskNoneFull); else TJK_OCC(bf16, 64, 64, kMaskNoneFull); }
+  else if (head_dim <= 96) { if (h16) TJK_OCC(f16, 128, 96, kMaskNoneFull); else TJK_OCC(bf16, 128, 96, kMaskNoneFull); }
+  else { if (h16) TJK_OCC(f16, 128, 128, kMaskNoneFull); else TJK_OCC(bf16, 128, 128, kMaskNoneFull); }
 #undef TJK_OCC
   if (e != hipSuccess) return fail(hip_status(e), "tjk_flash_sched_occupancy: %s", hipGetErrorString(e));
   return blocks;
