@@ -535,8 +535,6 @@ __global__ __launch_bounds__(64) void flash_short_kernel(
 // Cache-policy bits of buffer loads / stores (sc0 = 1, sc1 = 16): sc1 makes
 // an access device-coherent, sc0 sc1 on a store writes through to memory.
 constexpr int kFaSc1 = 16, kFaSc0Sc1 = 17;
-typedef __attribute__((address_space(3))) void lds_void;
-
 // Most keys a masked launch of the DMA ring can list (16 KB beside the 64 KB
 // ring of head_dim 64, two workgroups per CU).
 constexpr int kFaListKeys = 8064;
@@ -548,16 +546,6 @@ __device__ __forceinline__ u32x4 fa_rsrc(const void* p, int bytes) {
   const uint64_t a = (uint64_t)p;
   return u32x4{(uint32_t)a, (uint32_t)(a >> 32) & 0xffffu, (uint32_t)bytes, 0x00020000u};
 }
-// One LDS DMA: each lane copies 16 bytes at voff of the descriptor's range to
-// LDS byte lds_addr + 16 * lane.  Issued as inline asm so that the compiler
-// does not track it: for an LDS read it cannot tell apart from a DMA's
-// destination (the transposing ds_read_b64_tr_b16 carries no alias
-// information) it would otherwise wait for every copy in flight.  The ring's
-// own s_waitcnt vmcnt + s_barrier order the copies against the reads.
-__device__ __forceinline__ void fa_lds_dma16(u32x4 rsrc, uint32_t voff, uint32_t lds_addr) {
-  asm volatile("buffer_load_dwordx4 %0, %1, 0 offen lds" ::"v"(voff), "s"(rsrc), "{m0}"(lds_addr));
-}
-
 // NW waves per workgroup own BMQ = 32 NW queries.  NW = 4 (two workgroups
 // per CU at head_dim <= 64, one above).  NW = 8 is the head_dim-128 grid
 // variant: the LDS ring (143 KB) allows one workgroup per CU, so 8 waves
@@ -885,9 +873,9 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(HDP <= 
         off[q] = t * BNK + r < kend ? (uint32_t)dkey[q] * row_bytes + dvoff[q] : kPastRange;
       }
 #pragma unroll
-      for (int q = 0; q < NDK; ++q) fa_lds_dma16(rk, off[q], kb + q * NW * 1024);
+      for (int q = 0; q < NDK; ++q) lds_dma16(rk, off[q], kb + q * NW * 1024);
 #pragma unroll
-      for (int q = 0; q < NDK; ++q) fa_lds_dma16(rv, off[q], kb + TILE_B + q * NW * 1024);
+      for (int q = 0; q < NDK; ++q) lds_dma16(rv, off[q], kb + TILE_B + q * NW * 1024);
       next_keys(t + 1);
       return;
     }
@@ -896,9 +884,9 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(HDP <= 
     const u32x4 rsk = fa_rsrc(qbase + sc + t_elems, nrec), rsv = fa_rsrc(qbase + 2 * sc + t_elems, nrec);
     const uint32_t kb = lds_ring + (uint32_t)(st * 2 * TILE_B + wave * 1024);
 #pragma unroll
-    for (int q = 0; q < NDK; ++q) fa_lds_dma16(rsk, dvoff[q], kb + q * NW * 1024);
+    for (int q = 0; q < NDK; ++q) lds_dma16(rsk, dvoff[q], kb + q * NW * 1024);
 #pragma unroll
-    for (int q = 0; q < NDK; ++q) fa_lds_dma16(rsv, dvoff[q], kb + TILE_B + q * NW * 1024);
+    for (int q = 0; q < NDK; ++q) lds_dma16(rsv, dvoff[q], kb + TILE_B + q * NW * 1024);
   };
   // end of a ring step: this wave's copies of the tile two ahead have landed
   // (only the newest tile's may still be in flight) and its LDS reads are
@@ -1741,7 +1729,7 @@ extern "C" int tjk_flash_fwd(const void* qkv, int64_t stride_b, int64_t stride_s
   // length (causal 4 x 2048: 54 vs 60 us; S = 32768: 944 vs 790 TFLOP/s);
   // at hd 128 too since its 8-wave workgroups (causal 16 x 512: 50.5 vs
   // 53.0 us, 4 x 2048: 95.1 vs 122.6 us, 2 x 8192: 615 vs 743 us); plans 2
-  // and 3 were slower on every BASELINE shape.
+  // and 3 were slower on every benchmark configuration.
   // With a key mask plan 0 lists the admissible keys of 256 up to kFaListKeys
   // keys (flash_lists); otherwise it runs every tile through its masked
   // (unpipelined) loop, and past kFaListKeys plan 1 is faster (4 x 2048, hd 64:

@@ -519,8 +519,6 @@ template <int BKB> __device__ __forceinline__ int swz(int r);
 template <> __device__ __forceinline__ int swz<128>(int r) { return (r & 7) ^ ((r >> 3) & 1); }
 template <> __device__ __forceinline__ int swz<64>(int r) { return ((r >> 1) ^ (r >> 3)) & 3; }
 
-typedef __attribute__((address_space(3))) void lds_void;
-
 // Byte offset beyond any buffer descriptor range (those are signed 32-bit
 // counts); a row's offset inside a range added to it still fits 32 bits.
 constexpr uint32_t kPastEnd = 0x80000000u;
@@ -830,14 +828,6 @@ __device__ __forceinline__ u32x4 lds_dma_rsrc(const void* p, int64_t bytes) {
                (uint32_t)__builtin_amdgcn_readfirstlane((uint32_t)(a >> 32)) & 0xffffu,
                (uint32_t)__builtin_amdgcn_readfirstlane(n), 0x00020000u};
 }
-// One LDS DMA: each lane copies 16 bytes at voff of the descriptor's range
-// (zeros past it) to LDS byte lds_addr + 16 * lane.  Inline asm, so that the
-// compiler does not wait for copies in flight before LDS reads; the caller's
-// s_waitcnt vmcnt and s_barrier order them.
-__device__ __forceinline__ void lds_dma16(u32x4 rsrc, uint32_t voff, uint32_t lds_addr) {
-  asm volatile("buffer_load_dwordx4 %0, %1, 0 offen lds" ::"v"(voff), "s"(rsrc), "{m0}"(lds_addr));
-}
-
 // Waits until panel_accumulate's MFMAs have written their results.  The
 // compiler does not see an MFMA in inline asm: it neither inserts the wait
 // states before another instruction may read the result (8 for a 4-pass MFMA

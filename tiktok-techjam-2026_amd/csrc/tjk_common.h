@@ -303,4 +303,16 @@ __device__ __forceinline__ void wave_sum_n(float (&v)[N]) {
   }
 }
 
+typedef __attribute__((address_space(3))) void lds_void;
+
+// One LDS DMA: each lane copies 16 bytes at voff of the descriptor's range
+// (zeros past it) to LDS byte lds_addr + 16 * lane.  Inline asm, so that the
+// compiler does not track it: for an LDS read that it cannot tell apart from the
+// copy's destination (the transposing ds_read_b64_tr_b16 carries no alias
+// information) it would wait for every copy in flight.  The caller's s_waitcnt
+// vmcnt and s_barrier order the copies against the reads.
+__device__ __forceinline__ void lds_dma16(u32x4 rsrc, uint32_t voff, uint32_t lds_addr) {
+  asm volatile("buffer_load_dwordx4 %0, %1, 0 offen lds" ::"v"(voff), "s"(rsrc), "{m0}"(lds_addr));
+}
+
 }  // namespace tjk
