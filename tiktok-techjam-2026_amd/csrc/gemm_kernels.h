@@ -409,11 +409,11 @@ __global__ __launch_bounds__((WM * WN + L) * 64) void gemm_ws_kernel(
 // panel_accumulate's main loop (gemm_tiles.h) under the shared epilogue: four
 // waves, wave tile (32 FM) x (32 FN).  The same K order as the class-1 plans:
 // a 16x16x32 MFMA gives the bits of two 32x32x16 ones (tests compare every
-// plan of the class).  256 x 256 fills a CU (128 KB of LDS, 256 AGPRs); the
-// smaller tiles run two workgroups per CU, whose main loops cover each
-// other's prologue and epilogue.  Measured (bf16, one box, against the best
-// other plan): 8192^3 806 -> 709 us (plan 8), 8192 x 2048 x 8192 with the
-// residual 209 -> 184 us, 5430 x 4096 x 1024 with GELU 56.0 -> 51.5 us (192 x
+// plan of the class).  256 x 256 fills a CU (128 KB of LDS, 256 AGPRs, nothing in
+// scratch); the smaller tiles run two workgroups per CU, whose main loops cover
+// each other's prologue and epilogue.  Measured (bf16, one box, against the best
+// other plan): 8192^3 825 -> 715 us (plan 8), 8192 x 2048 x 8192 with the
+// residual 219 -> 190 us (8), 5430 x 4096 x 1024 with GELU 53.0 -> 50.1 us (192 x
 // 128 tiles; plan 31).  192 x 256, 256 x 128 and 192 x 192 tiles of this
 // kernel were no faster than these on any shape tried.
 template <typename T, int FM, int FN, int EPI>

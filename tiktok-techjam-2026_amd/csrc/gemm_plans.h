@@ -18,14 +18,15 @@ struct GemmPlan {
 
 // 2-byte types (bf16/fp16), BK = 64.  Which one a launch takes by default is
 // gemm.hip's estimate (kAuto16); `eff` only ranks the plans where no estimated
-// tile's offsets reach the rows.  (A 4-stage ring of 64-byte rows was tried and dropped: it
-// measured 50% LDS bank-conflict cycles and no gain.)
+// tile's offsets reach the rows, which leaves the staged ones (0-5).  (A 4-stage
+// ring of 64-byte rows was tried and dropped: it measured 50% LDS bank-conflict
+// cycles and no gain.)
 static const GemmPlan kPlans16[] = {
     {kStaged, 256, 256, 2, 2, 128, 2, 0.50},  // 0
     {kStaged, 256, 128, 2, 2, 128, 2, 0.45},  // 1
     {kStaged, 128, 256, 2, 2, 128, 2, 0.45},  // 2
     {kStaged, 128, 128, 2, 2, 128, 2, 0.55},  // 3
-    {kStaged, 64, 64, 2, 2, 128, 2, 0.40},    // 4  small shapes / K % 64 != 0
+    {kStaged, 64, 64, 2, 2, 128, 2, 0.40},    // 4
     {kStaged, 256, 256, 2, 4, 128, 2, 0.55},  // 5
     {kDtl, 256, 256, 2, 2, 128, 2, 0.85},     // 6  wave tile 128x128, 1 WG/CU
     {kDtl, 128, 128, 2, 2, 128, 2, 0.90},     // 7  wave tile 64x64, 2 WG/CU

@@ -766,8 +766,10 @@ __device__ __forceinline__ void dtl_accumulate(
 // Main loop for the largest tiles: 2 x 2 waves with (32 FM) x (32 FN) wave
 // tiles, one wave per SIMD, accumulators in all 256 AGPRs (FM = FN = 4).
 // What bounds these launches on MI355X is power: the matrix pipe is busy
-// ~90% of the main loop's cycles while the clock sits at 1.5-1.7 GHz, so the
-// loop is built to spend less energy per product and to keep the pipe fed:
+// ~90% of the main loop's cycles while the clock sits at 1.5-1.7 GHz (8192^3: 2303
+// cycles per K tile by the clock counter, 2048 of them MFMA, 512 K tiles per CU
+// in 715 us), so the loop is built to spend less energy per product and to keep
+// the pipe fed:
 //   * 16x16x32 MFMAs: one instruction contracts 32 of K, so an accumulator
 //     is read and written half as often per product as with 32x32x16.  The
 //     MFMAs alone ran at 2.19 GHz against 1.89 GHz (same probe, 256 x 256

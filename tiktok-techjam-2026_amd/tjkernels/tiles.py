@@ -27,7 +27,8 @@ and the four-way split when one round of 32 x 64 tiles covers the launch and
 K >= 2048 (C2's FFN2).  In fp32 the four-way split takes launches of up to 128
 tiles of 64 x 64 (192 with K >= 2048), else class 1.  The library's own rule
 (k_class in csrc/gemm.hip) is the same, so a launch without a plan keeps these
-classes too.
+classes too (``tjk_gemm_default_plan``), but for row pitches past the tiles' 31-bit
+offsets, which it takes in class 1.
 
 The LayerNorm-prologue GEMM (``tjk_gemm_ln``, LayerNorm computed inside
 the GEMM for launch-bound row counts) has its own plans, 32-row tiles of
