@@ -535,6 +535,7 @@ __global__ __launch_bounds__(64) void flash_short_kernel(
 // Cache-policy bits of buffer loads / stores (sc0 = 1, sc1 = 16): sc1 makes
 // an access device-coherent, sc0 sc1 on a store writes through to memory.
 constexpr int kFaSc1 = 16, kFaSc0Sc1 = 17;
+
 // Most keys a masked launch of the DMA ring can list (16 KB beside the 64 KB
 // ring of head_dim 64, two workgroups per CU).
 constexpr int kFaListKeys = 8064;
@@ -546,6 +547,7 @@ __device__ __forceinline__ u32x4 fa_rsrc(const void* p, int bytes) {
   const uint64_t a = (uint64_t)p;
   return u32x4{(uint32_t)a, (uint32_t)(a >> 32) & 0xffffu, (uint32_t)bytes, 0x00020000u};
 }
+
 // NW waves per workgroup own BMQ = 32 NW queries.  NW = 4 (two workgroups
 // per CU at head_dim <= 64, one above).  NW = 8 is the head_dim-128 grid
 // variant: the LDS ring (143 KB) allows one workgroup per CU, so 8 waves
@@ -560,7 +562,7 @@ __device__ __forceinline__ u32x4 fa_rsrc(const void* p, int bytes) {
 // of a row from head_dim on are copied from outside the buffer range: zeros.
 // Measured against the register-staged ring that served every head_dim but 64
 // and 128 before (128 columns computed at 96): 4 x 2048 x 16 heads of 96, bf16
-// causal, 77.8 -> 65.9 us, with a key mask 214 -> 63, of 32 with a key mask 72
+// causal, 84.3 -> 67.7 us, with a key mask 214 -> 63, of 32 with a key mask 72
 // -> 39.  Without one, head dims 8, 16 and 40 gain 0-11%, 72 to 96 11-17%; 24, 48
 // and 56 gain up to 11% and lose up to 13% (24) and 9% by the shape, 104 to 120
 // gain or lose 4%; head_dim 32 keeps its registers (PipeFull).
@@ -600,8 +602,7 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(HDP <= 
   // lds, K and V both key-major with 128- / 256-byte rows whose 16-byte chunks
   // are XOR-swizzled by row, and V^T fragments are gathered with the
   // transposing ds_read_b64_tr_b16.  Otherwise (a key mask that is not listed,
-  // head_dim 32) tiles pass through registers, V stored
-  // transposed.
+  // head_dim 32) tiles pass through registers, V stored transposed.
   constexpr bool FULLHD = MASK == kMaskBytesFull || MASK == kMaskNoneRegs || MASK == kMaskNoneFull;
   constexpr bool KEYMASK = MASK == kMaskBytes || MASK == kMaskBytesFull, DMA = !KEYMASK && MASK != kMaskNoneRegs;
   static_assert(!DMA || HDP >= 64, "rows of whole 8-chunk XOR groups");
@@ -611,9 +612,9 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(HDP <= 
   // masked keys cost nothing.  Key limits (kend, lim, ...) then count listed
   // keys.  Before, every tile of a masked launch loaded 32 mask bytes per lane
   // and ran the unpipelined loop.  Measured with a quarter of the keys masked:
-  // 8 x 512 x 12 heads of 64, fp16, 29.4 -> 19.2 us (15.3 without a mask); 4 x
-  // 2048 x 16 heads of 64, bf16 causal, 109 (plan 1) -> 55 us (48); 2 x 4096 x
-  // 16 heads of 128, causal, 408 -> 122 us (132).
+  // 8 x 512 x 12 heads of 64, fp16, 29.7 -> 18.4 us (15.4 without a mask); 4 x
+  // 2048 x 16 heads of 64, bf16 causal, 109 (plan 1) -> 54 us (47); 2 x 4096 x
+  // 16 heads of 128, causal, 410 -> 120 us (135).
   constexpr bool LIST = MASK == kMaskList;
   constexpr int RB = HDP * (int)sizeof(T);  // DMA: bytes per K / V row
   constexpr int CPR = RB / 16, RPI = 64 / CPR, TILE_B = BNK * RB;
@@ -979,8 +980,7 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(HDP <= 
   // P, as in flash_fwd_kernel, which ran masked launches of 2048 keys and more
   // before (error against 64 bits, bf16 causal 1 x 4096 x 2 heads of 64: 2.03e-3
   // there, 2.08e-3 with the lazy offset, 2.02e-3 so; scores 4 times as spread
-  // 1.73, 1.86 and 1.73e-3).  It costs 8 x 512 x 12 heads of 64, fp16, 17.0 ->
-  // 18.5 us, 4 x 2048 x 16 causal 48 -> 54.
+  // 1.73, 1.86 and 1.73e-3).  It costs 7-12% of the launch.
   constexpr float kLazyRescale = LIST ? 0.f : 8.0f;
   float m_off = -INFINITY, l_run = 0.f;
 
